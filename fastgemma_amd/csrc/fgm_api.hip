@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1037,7 +1038,7 @@ void fgm_softcap_hip(float* x, int n, float cap) { DROPIN(dropin_softcap(x, n, c
 // Validates the sequences, fills the row bookkeeping and the grid of `a`
 // (scratch pointers excepted); *max_n, *max_span receive the longest range
 // and the longest range-or-ring of any row.
-static int attn_plan(AttnArgs& a, int* max_n, int* max_span) {
+static int attn_plan(AttnArgs& a, int* max_span) {
   if (a.nh <= 0 || a.kvh <= 0 || a.nh % a.kvh)
     return fail(FGM_HIP_EINVAL, "attend: n_heads=%d is not a multiple of kv_heads=%d", a.nh, a.kvh);
   if (a.nh / a.kvh > 16) return fail(FGM_HIP_EINVAL, "attend: %d query heads per kv head > 16", a.nh / a.kvh);
@@ -1051,6 +1052,7 @@ static int attn_plan(AttnArgs& a, int* max_n, int* max_span) {
   if (!a.out || !a.q) return fail(FGM_HIP_EINVAL, "attend: out or q is NULL");
   int m = 0, mn = 0, ms = 1, p1max = 1, steps_max = 1;
   long long tiles = 0;
+  std::fill(a.row0, a.row0 + FGM_ATTN_MAX_SEQ, INT_MAX);
   for (int i = 0; i < a.nseq; i++) {
     AttnSeq& s = a.seq[i];
     if (s.nrows < 0) return fail(FGM_HIP_EINVAL, "attend: sequence %d has %d rows", i, s.nrows);
@@ -1058,10 +1060,12 @@ static int attn_plan(AttnArgs& a, int* max_n, int* max_span) {
       return fail(FGM_HIP_EINVAL, "attend: sequence %d has a NULL cache pointer", i);
     if (s.k_len <= 0 || s.ring < 0 || s.ring > s.k_len)
       return fail(FGM_HIP_EINVAL, "attend: sequence %d: k_len=%d ring=%d", i, s.k_len, s.ring);
-    s.row0 = m;
+    s.row0 = a.row0[i] = m;
     m += s.nrows;
     for (int j = 0; j < s.nrows; j++) {
-      const AttnSpan sp = attn_span(s.pos0 + j + 1, s.lo, a.window, s.ring);
+      const AttnSpan sp = attn_span(s.pos0 + j + 1, s.lo, a.window, s.ring,
+                                    [&](int st) { return s.ring ? st % s.ring : st; });
+      if (j == 0) s.st0 = sp.st, s.slot0 = sp.s0;
       if (sp.st < 0 || sp.n < 0)
         return fail(FGM_HIP_EINVAL, "attend: sequence %d row %d: range [%d,%d)", i, j, sp.st, sp.en);
       if (!s.ring && sp.en > s.k_len)
@@ -1088,21 +1092,24 @@ static int attn_plan(AttnArgs& a, int* max_n, int* max_span) {
   // P.V: the row's 64-slot steps split into at most attn_pv_chunks chunks
   const int chunks = m ? attn_pv_chunks(m, a.kvh, a.hd) : 1;
   a.p3_spw = std::max(1, (steps_max + 4 * chunks - 1) / (4 * chunks));
-  *max_n = mn;
+  a.one_row = 1;
+  for (int i = 0; i < a.nseq; i++) a.one_row &= a.seq[i].nrows == 1;
+  a.max_n = mn;
+  a.max_steps = steps_max;
   *max_span = ms;
   return FGM_HIP_OK;
 }
 
 static int attn_run(AttnArgs& a, void* scratch, size_t scratch_bytes, hipStream_t st) {
-  int max_n, max_span, rc;
-  if ((rc = attn_plan(a, &max_n, &max_span))) return rc;
+  int max_span, rc;
+  if ((rc = attn_plan(a, &max_span))) return rc;
   if (a.m == 0 || a.h0 == a.h1) return FGM_HIP_OK;
   const size_t need = fgm_attn_layout(nullptr, nullptr, a.m, a.nh, a.kvh, a.hd, max_span);
   if (!scratch || scratch_bytes < need)
     return fail(FGM_HIP_EINVAL, "attend: scratch of %zu bytes, this call needs %zu", scratch_bytes, need);
   if (((uintptr_t)scratch) & 255) return fail(FGM_HIP_EINVAL, "attend: scratch must be 256-byte aligned");
   fgm_attn_layout(&a, scratch, a.m, a.nh, a.kvh, a.hd, max_span);
-  hipError_t e = fgm_launch_attn(a, max_n, st);
+  hipError_t e = fgm_launch_attn(a, st);
   return e == hipSuccess ? FGM_HIP_OK : hip_fail(e, "attention launch");
 }
 
@@ -1121,7 +1128,7 @@ int fgm_hip_attend_dev(float* out, const float* q, const fgm_hip_attn_seq* seqs,
   AttnArgs a{};
   for (int i = 0; i < nseq; i++) {
     const fgm_hip_attn_seq& s = seqs[i];
-    a.seq[i] = AttnSeq{s.kc, s.ks, s.vc, s.vs, s.k_len, s.ring, s.pos, 0, s.rows, 0};
+    a.seq[i] = AttnSeq{s.kc, s.ks, s.vc, s.vs, s.k_len, s.ring, s.pos, 0, s.rows, 0, 0, 0};
   }
   a.nseq = nseq, a.nh = n_heads, a.kvh = kv_heads, a.hd = head_dim, a.window = window;
   a.h0 = 0, a.h1 = n_heads, a.out = out, a.q = q;
@@ -1137,7 +1144,7 @@ int fgm_hip_attend_heads_dev(float* out, const float* q, const int8_t* kc, const
   if (start < 0 || end < start)
     return fail(FGM_HIP_EINVAL, "attend_heads: range [%d,%d)", start, end);
   AttnArgs a{};
-  a.seq[0] = AttnSeq{kc, ks, vc, vs, cap, ring, end - 1, start, 1, 0};
+  a.seq[0] = AttnSeq{kc, ks, vc, vs, cap, ring, end - 1, start, 1, 0, 0, 0};
   a.nseq = 1, a.nh = n_heads, a.kvh = kv_heads, a.hd = head_dim, a.window = 0;
   a.h0 = h0, a.h1 = h1, a.out = out, a.q = q;
   return attn_run(a, scratch, scratch_bytes, (hipStream_t)stream);
@@ -1179,9 +1186,9 @@ static int dropin_attend(float* out, const float* q, const int8_t* kc, const flo
   if (n_heads <= 0 || kv_heads <= 0 || head_dim <= 0 || cap <= 0 || h1 <= h0) {
     AttnArgs a{};
     a.nh = n_heads, a.kvh = kv_heads, a.hd = head_dim, a.h0 = h0, a.h1 = h1;
-    int mn, ms;
+    int ms;
     a.out = out, a.q = q;
-    return attn_plan(a, &mn, &ms);  // reports the invalid argument, or nothing to do
+    return attn_plan(a, &ms);  // reports the invalid argument, or nothing to do
   }
   const size_t kvd = (size_t)kv_heads * head_dim;
   const size_t kb = (size_t)cap * kvd, vb = (size_t)(cap + 3) / 4 * 4 * kvd, ob = (size_t)n_heads * head_dim * 4;

@@ -36,10 +36,24 @@
 
 namespace {
 
+// max over each row of 16 lanes
+FGM_DEV float row16_max(float v) {
+  v = __builtin_fmaxf(v, row_ror<8>(v));
+  v = __builtin_fmaxf(v, row_ror<4>(v));
+  v = __builtin_fmaxf(v, row_ror<2>(v));
+  return __builtin_fmaxf(v, row_ror<1>(v));
+}
+
+// max over the wave, in every lane (DPP row broadcasts: no LDS round trips)
 FGM_DEV float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = __builtin_fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  v = row16_max(v);
+  auto bcast = [&](auto ctrl) {
+    const int i = __float_as_int(v);
+    v = __builtin_fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(i, i, decltype(ctrl)::value, 0xF, 0xF, false)));
+  };
+  bcast(std::integral_constant<int, 0x142>{});  // lane 15 of each row to the next row
+  bcast(std::integral_constant<int, 0x143>{});  // lane 31 to the upper half
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
 // max over the workgroup; `red` holds one float per wave; every thread gets it
@@ -61,34 +75,100 @@ struct Geo {
   const int8_t* vc;
   const float* vs;
   int k_len, ring, st, en, n;
-  int nrun, lo0, hi0, lo1, hi1;
-  int dom_lo, dom_steps;  // slot domain of the P.V kernel: [dom_lo, dom_lo + 64 dom_steps)
+  int s0;                           // slot of position st
+  int lo0, hi1;                     // slots [lo0, hi1) lie in both spans (none when lo0 >= hi1)
+  int dom_lo, dom_steps, nst1, gap; // slot domain of P.V: see AttnSpan
+
+  __device__ int slot_of(int u) const {  // position st + u, u < n
+    const int s = s0 + u;
+    return ring && s >= ring ? s - ring : s;
+  }
+  // u of the position held in slot s of the range, outside [0, n) if none
+  __device__ int pos_of(int s) const {
+    if (ring && s >= ring) return -1;
+    const int u = s - s0;
+    return u < 0 ? u + ring : u;
+  }
+  // offset of slot s in the P.V domain
+  __device__ int dom_off(int s) const {
+    const int d = s - dom_lo;
+    return d >= 64 * nst1 + gap ? d - gap : d;
+  }
+  __device__ bool twice(int s) const { return s >= lo0 && s < hi1; }
+  __device__ int dom_slot(int step) const { return dom_lo + 64 * step + (step >= nst1 ? gap : 0); }
+  __device__ int dom_slot4(int qd) const { return dom_lo + 4 * qd + ((qd >> 4) >= nst1 ? gap : 0); }
 };
 
 FGM_DEV Geo row_geo(const AttnArgs& a, int r) {
-  // the sequence holding row r, selected field by field (no dynamic index
-  // into the kernel argument)
-  const int8_t* kc = a.seq[0].kc;
-  const float* ks = a.seq[0].ks;
-  const int8_t* vc = a.seq[0].vc;
-  const float* vs = a.seq[0].vs;
-  int k_len = a.seq[0].k_len, ring = a.seq[0].ring, pos0 = a.seq[0].pos0, lo = a.seq[0].lo,
-      row0 = a.seq[0].row0;
+  // the sequence holding row r: one sequence, or one row each, need no look
+  // at the row table (a dependent fetch of the arguments less); its fields by
+  // that (uniform) index from the kernel argument itself
+  int i = 0;
+  if (a.one_row) {
+    i = r;
+  } else if (a.nseq > 1) {
 #pragma unroll
-  for (int j = 1; j < FGM_ATTN_MAX_SEQ; j++) {
-    if (j < a.nseq && r >= a.seq[j].row0) {
-      kc = a.seq[j].kc, ks = a.seq[j].ks, vc = a.seq[j].vc, vs = a.seq[j].vs;
-      k_len = a.seq[j].k_len, ring = a.seq[j].ring, pos0 = a.seq[j].pos0, lo = a.seq[j].lo;
-      row0 = a.seq[j].row0;
-    }
+    for (int j = 1; j < FGM_ATTN_MAX_SEQ; j++) i += r >= a.row0[j];
   }
-  const AttnSpan sp = attn_span(pos0 + (r - row0) + 1, lo, a.window, ring);
+  const auto* ka = (const __attribute__((address_space(4))) AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  const auto& s = ka->seq[__builtin_amdgcn_readfirstlane(i)];
   Geo g;
-  g.kc = kc, g.ks = ks, g.vc = vc, g.vs = vs, g.k_len = k_len, g.ring = ring;
-  g.st = sp.st, g.en = sp.en, g.n = sp.n, g.nrun = sp.nrun;
-  g.lo0 = sp.lo0, g.hi0 = sp.hi0, g.lo1 = sp.lo1, g.hi1 = sp.hi1;
-  g.dom_lo = sp.dom_lo, g.dom_steps = sp.dom_steps;
+  g.kc = s.kc, g.ks = s.ks, g.vc = s.vc, g.vs = s.vs, g.k_len = s.k_len, g.ring = s.ring;
+  const int dr = r - s.row0;
+  const AttnSpan sp = attn_span(s.pos0 + dr + 1, s.lo, a.window, g.ring, [&](int st) {
+    // the slot of the sequence's first row's start is known: no division
+    // unless the rows run past the ring
+    int s0 = s.slot0 + (st - s.st0);
+    if (g.ring && s0 >= g.ring) s0 = s0 < 2 * g.ring ? s0 - g.ring : s0 % g.ring;
+    return s0;
+  });
+  g.st = sp.st, g.en = sp.en, g.n = sp.n, g.s0 = sp.s0;
+  g.lo0 = sp.lo0, g.hi1 = sp.hi1;
+  g.dom_lo = sp.dom_lo, g.dom_steps = sp.dom_steps, g.nst1 = sp.nst1, g.gap = sp.gap;
   return g;
+}
+
+// The reference's sum of exponentials over the 16-wide chunks, for lanes
+// 0..15 of one wave (lane j: c = row j of the transposed row, e[16 t + j] at
+// c[t], 16 readable floats past nt): lane j sums its column in chunk order,
+// reads two groups ahead, then _mm512_reduce_add_ps on DPP row rotations.
+FGM_DEV float chunk_sum16(const float* c, int nt) {
+  float acc = 0.0f;
+  float4 P[4], Q[4];
+  auto rd = [&](float4* p, int t0) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) p[q] = *(const float4*)(c + t0 + 4 * q);
+  };
+  auto add = [&](const float4* p) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      acc = acc + p[q].x;
+      acc = acc + p[q].y;
+      acc = acc + p[q].z;
+      acc = acc + p[q].w;
+    }
+  };
+  int t = 0;
+  rd(P, 0);
+  for (; t + 32 <= nt; t += 32) {
+    rd(Q, t + 16);
+    __builtin_amdgcn_sched_barrier(0);
+    add(P);
+    __builtin_amdgcn_sched_barrier(0);
+    rd(P, t + 32);
+    __builtin_amdgcn_sched_barrier(0);
+    add(Q);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (t + 16 <= nt) {
+    add(P);
+    t += 16;
+  }
+  for (; t < nt; t++) acc = acc + c[t];
+  acc = acc + row_ror<8>(acc);
+  acc = acc + row_ror<4>(acc);
+  acc = acc + row_ror<2>(acc);
+  return acc + row_ror<1>(acc);
 }
 
 // ------------------------------------------------------------- 1. scores
@@ -117,8 +197,8 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(const AttnArgs a) {
   // quantised)
   auto load = [&](v4i* B, float& kscale, int t0) {
     const int t = t0 + (lane & 15);
-    const int slot = G.ring ? t % G.ring : t;
     const bool ok = t < t_end;
+    const int slot = ok ? G.slot_of(t - G.st) : 0;
     const uint32_t base = ok ? (uint32_t)slot * (uint32_t)kvd + (uint32_t)(g * HD + 16 * (lane >> 4)) : FGM_OOB;
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) B[kk] = buf_load_b128(rk, base, 64 * kk);
@@ -219,46 +299,7 @@ __global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
   }
   __syncthreads();
   if (tid < 16) {
-    // lane j: e[16 c + j] summed in chunk order, reads two groups ahead
-    const int nt = n16 >> 4;
-    const float* c = lds + tid * S;
-    float acc = 0.0f;
-    float4 P[4], Q[4];
-    auto rd = [&](float4* p, int t0) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) p[q] = *(const float4*)(c + t0 + 4 * q);
-    };
-    auto add = [&](const float4* p) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        acc = acc + p[q].x;
-        acc = acc + p[q].y;
-        acc = acc + p[q].z;
-        acc = acc + p[q].w;
-      }
-    };
-    int t = 0;
-    rd(P, 0);
-    for (; t + 32 <= nt; t += 32) {
-      rd(Q, t + 16);
-      __builtin_amdgcn_sched_barrier(0);
-      add(P);
-      __builtin_amdgcn_sched_barrier(0);
-      rd(P, t + 32);
-      __builtin_amdgcn_sched_barrier(0);
-      add(Q);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (t + 16 <= nt) {
-      add(P);
-      t += 16;
-    }
-    for (; t < nt; t++) acc = acc + c[t];
-    // _mm512_reduce_add_ps
-    acc = acc + row_ror<8>(acc);
-    acc = acc + row_ror<4>(acc);
-    acc = acc + row_ror<2>(acc);
-    float sum = acc + row_ror<1>(acc);
+    float sum = chunk_sum16(lds + tid * S, n16 >> 4);
     if (tid == 0) {
       for (int u = n16; u < n; u++) sum += lds[(u & 15) * S + (u >> 4)];
       red[nw] = 1.0f / sum;
@@ -273,8 +314,8 @@ __global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
     float vsv[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-      const int u = b + j * T, t = G.st + u;
-      vsv[j] = u < n ? G.vs[G.ring ? t % G.ring : t] : 0.0f;
+      const int u = b + j * T;
+      vsv[j] = u < n ? G.vs[G.slot_of(u)] : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < 8; j++) {
@@ -293,36 +334,23 @@ __global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
 
   // weight planes for every slot of the P.V domain, four slots per thread
   int8_t* wp = a.wpl + (size_t)(r * a.kvh + g) * a.wpl_blocks * (48 * grp) + hl * 16;
-  const int dom_hi = G.dom_lo + 64 * G.dom_steps;
-  for (int s4 = G.dom_lo + 4 * tid; s4 < dom_hi; s4 += 4 * T) {
+  for (int qd = tid; qd < 16 * G.dom_steps; qd += T) {
+    const int s4 = G.dom_slot4(qd);
     uint32_t pa = 0, pb = 0, pc = 0;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      const int s = s4 + e;
+      const int u = G.pos_of(s4 + e);
       int W = 0;
-      const int mult = (s >= G.lo0 && s < G.hi0) + (G.nrun == 2 && s >= G.lo1 && s < G.hi1);
-      if (pos && mult) {
-        int t;
-        bool ok;
-        if (!G.ring) {
-          t = s, ok = s >= G.st && s < G.en;
-        } else {  // the latest position of the range held in slot s
-          const int d = ((G.en - 1 - s) % G.ring + G.ring) % G.ring;
-          t = G.en - 1 - d, ok = s < G.ring && t >= G.st;
-        }
-        if (ok) {
-          const int u = t - G.st;
-          const float wt = lds[(u & 15) * S + (u >> 4)];
-          int q = (int)__builtin_fmaf(wt, wq_inv, 0.5f);
-          q = q > 65535 ? 65535 : (q < 0 ? 0 : q);
-          W = mult * q;
-        }
+      if (pos && (unsigned)u < (unsigned)n) {
+        int q = (int)__builtin_fmaf(lds[(u & 15) * S + (u >> 4)], wq_inv, 0.5f);
+        q = q > 65535 ? 65535 : (q < 0 ? 0 : q);
+        W = G.twice(s4 + e) ? 2 * q : q;
       }
       pa |= (uint32_t)(W >> 14) << (8 * e);
       pb |= (uint32_t)((W >> 7) & 127) << (8 * e);
       pc |= (uint32_t)(W & 127) << (8 * e);
     }
-    int8_t* p = wp + (size_t)((s4 - G.dom_lo) >> 4) * (48 * grp) + (s4 & 15);
+    int8_t* p = wp + (size_t)(qd >> 2) * (48 * grp) + 4 * (qd & 3);
     *(uint32_t*)p = pa;
     *(uint32_t*)(p + 16 * grp) = pb;
     *(uint32_t*)(p + 32 * grp) = pc;
@@ -361,8 +389,8 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(const AttnArgs a) {
   // A: plane p, row hl, the 16 slots s0 + 16 q4 + [0, 16); B: dim
   // d0 + 16 nt + hl, dword q = the four slots of group s0 / 4 + 4 q4 + q
   auto load = [&](v4i* A, int* B, int step) {
-    const int s0 = G.dom_lo + 64 * step;
-    const int8_t* wp = wrow + (size_t)(((s0 - G.dom_lo) >> 4) + q4) * (48 * grp);
+    const int s0 = G.dom_slot(step);
+    const int8_t* wp = wrow + (size_t)(4 * step + q4) * (48 * grp);
 #pragma unroll
     for (int p = 0; p < 3; p++) A[p] = live ? *(const v4i*)(wp + p * 16 * grp) : v4i{0, 0, 0, 0};
 #pragma unroll
@@ -436,65 +464,91 @@ __global__ __launch_bounds__(64) void attn_final_kernel(const AttnArgs a) {
 
 // ------------------------------------------------------ single-launch path
 // Rows of at most FUSED_MAX_N positions and kv groups of at most 8 query
-// heads: one workgroup per (row, kv head) does all four steps above with the
-// same arithmetic, the scores, exponentials and weight planes in LDS and the
-// P.V sums in registers -- one launch instead of four (sliding-window layers,
-// short contexts).  grid (m * kvh), 512 threads; dynamic LDS:
-//   qq [16][hd + 16] int8 | qsc, wqs, winv [16] f32 |
-//   E [grp][16][S] f32 (per head, e[16 c + j] at [j][c]) |
-//   planes [blocks][3][grp][16] int8.
-constexpr int FUSED_MAX_N = 1024, FUSED_MAX_GRP = 8, FUSED_T = 512, FUSED_NW = FUSED_T / 64;
+// heads: one workgroup per (row, kv head, hpw of its query heads) does all
+// four steps above with the same arithmetic, the scores, exponentials and
+// weight planes in LDS and the P.V sums in registers -- one launch instead of
+// four (sliding-window layers, short contexts).  A launch of a few rows is one
+// dependent chain (arguments, K, softmax, P.V, each a few hundred
+// instructions, fetched cold), so its heads are dealt to separate workgroups
+// until they fill the chip (each reads the K and V of its kv head again, from
+// the L2 of its XCD), and the softmax runs one position per lane in loops that
+// are not unrolled.  8 rows x 8 heads x 512 positions at head_dim 256: 22.8 us
+// with the eight heads in one workgroup of eight waves, 11.4 us split and
+// walked this way; 256 rows (every head in one workgroup of sixteen waves)
+// 22.2 -> 15.0 us.  Of the 11.4, 2.2 us pass before the wait for the first
+// K and query bytes ends, 2 us more in that wait.  grid (HS, m * kvh) flattened with the row fastest (the
+// workgroups of one row land on one XCD when the rows are a multiple of 8);
+// 64 NW threads; dynamic LDS:
+//   qq [16][hd + 16] int8 | qsc, wqs [16] f32 | smax [8][16] f32 | wred [16] f32 |
+//   E [hpw][16][S] f32 (per head, e[16 c + j] at [j][c]), reused for the
+//   int32 P.V sums [NW][3 hpw][64] | planes [blocks][3 hpw][16] int8 + one row pad.
+constexpr int FUSED_MAX_N = 1024, FUSED_MAX_GRP = 8;
+// sixteen waves while a tile's registers leave room for four waves per SIMD
+// (eight: the decode job above the same, 256 rows 15.1 -> 15.5 us)
+__host__ __device__ constexpr int fused_waves(int hd) { return hd <= 256 ? 16 : 8; }
 
-__host__ __device__ inline size_t fused_lds(int hd, int grp, int max_n, int blocks) {
-  const int S = (((max_n + 15) >> 4) + 16 + 63) / 64 * 64 + 4;
-  return (size_t)16 * (hd + 16) + 48 * 4 + (size_t)grp * 16 * S * 4 + (size_t)blocks * 48 * grp;
+__host__ __device__ inline int fused_stride(int n) { return (((n + 15) >> 4) + 16 + 63) / 64 * 64 + 4; }
+__host__ __device__ inline size_t fused_e_bytes(int nw, int hpw, int max_n) {
+  const size_t e = (size_t)hpw * 16 * fused_stride(max_n) * 4, red = (size_t)nw * 3 * hpw * 64 * 4;
+  return e > red ? e : red;
+}
+// the last block's operand reads run to row 31 of 16 bytes
+inline size_t fused_lds(int nw, int hd, int hpw, int max_n, int steps) {
+  return (size_t)16 * (hd + 16) + (32 + 128 + 16) * 4 + fused_e_bytes(nw, hpw, max_n) +
+         (size_t)steps * 4 * 48 * hpw + 32 * 16;
 }
 
-template <int KS>
-__global__ __launch_bounds__(FUSED_T) void attn_fused_kernel(const AttnArgs a) {
-  constexpr int HD = KS * 64, QROW = HD + 16, NW = FUSED_NW;
+template <int KS, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_fused_kernel(const AttnArgs a) {
+  constexpr int HD = KS * 64, QROW = HD + 16;
+  constexpr int NSL = NW / KS;  // slot slices of the P.V product
   extern __shared__ __attribute__((aligned(16))) char sm[];
-  const int r = blockIdx.x / a.kvh, g = blockIdx.x - r * a.kvh;
+  const int rows = a.m * a.kvh, hs = blockIdx.x / rows, rg = blockIdx.x - hs * rows;
+  const int r = rg / a.kvh, g = rg - r * a.kvh;
   const Geo G = row_geo(a, r);
-  const int grp = a.nh / a.kvh;
-  const int hb = max(a.h0, g * grp), he = min(a.h1, (g + 1) * grp);
+  const int grp = a.nh / a.kvh, hpw = a.hpw;
+  // heads [hf, hf + nhl) of this workgroup; of them [h0, h1) are computed
+  const int hf = g * grp + hs * hpw, nhl = min(hpw, grp - hs * hpw);
+  const int hb = max(a.h0, hf), he = min(a.h1, hf + nhl);
   if (hb >= he) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int n = max(G.n, 0), n16 = n & ~15, S = exp_stride(n);
+  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+  const int n = max(G.n, 0), n16 = n & ~15, S = fused_stride(n);
   int8_t* qq = (int8_t*)sm;
   float* qsc = (float*)(sm + 16 * QROW);
-  float* wqs = qsc + 16;   // per head: wmax / 65535, 0 = zero output
-  float* winv = wqs + 16;  // per head: 1 / sum, then 65535 / wmax
-  float* E = winv + 16;
-  int8_t* PL = (int8_t*)(E + (size_t)grp * 16 * S);
+  float* wqs = qsc + 16;    // per head: wmax / 65535, 0 = zero output
+  float* smax = wqs + 16;   // [head][wave]: the maximum score
+  float* wred = smax + 128; // per wave: the maximum weight of its head
+  float* E = wred + 16;
+  int8_t* PL = (int8_t*)E + fused_e_bytes(NW, hpw, a.max_n);
   const int kvd = a.kvh * HD;
-  auto live_head = [&](int hl) { return hl < grp && g * grp + hl >= hb && g * grp + hl < he; };
+  const int c16 = lane & 15, q4 = lane >> 4;
 
-  // ---- scores: the first tile's K in flight while the query is quantised
+  // ---- K: position tiles of 16, wave w the tiles w, w + NW, ...; the first
+  // two in flight while the query is quantised
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(G.kc, (uint32_t)((size_t)G.k_len * kvd));
-  auto load = [&](v4i* B, float& kscale, int t0) {
-    const int t = t0 + (lane & 15);
-    const int slot = G.ring ? t % G.ring : t;
-    const bool ok = t < G.en;
-    const uint32_t base = ok ? (uint32_t)slot * (uint32_t)kvd + (uint32_t)(g * HD + 16 * (lane >> 4)) : FGM_OOB;
+  const __amdgpu_buffer_rsrc_t rks = make_rsrc(G.ks, (uint32_t)G.k_len * 4u);
+  auto load = [&](v4i* B, int& kscale, int u0) {
+    const int u = u0 + c16;
+    const int slot = G.slot_of(u);
+    const uint32_t base = u < n ? (uint32_t)slot * (uint32_t)kvd + (uint32_t)(g * HD + 16 * q4) : FGM_OOB;
+    kscale = buf_load_b32(rks, u < n ? 4u * (uint32_t)slot : FGM_OOB, 0);
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) B[kk] = buf_load_b128(rk, base, 64 * kk);
-    kscale = ok ? G.ks[slot] : 0.0f;
   };
   v4i B0[KS], B1[KS];
-  float ks0 = 0.0f, ks1 = 0.0f;
-  int t0 = G.st + 16 * w;
-  if (t0 < G.en) load(B0, ks0, t0);
-  for (int hl = w; hl < 16; hl += NW) {
-    const int h = g * grp + hl;
-    const bool live = live_head(hl);
+  int ks0 = 0, ks1 = 0;
+  int u0 = 16 * w;
+  // the int8 query, one wave per head; the rows of A past nhl hold whatever
+  // LDS held, and so do the scores' rows that nobody reads
+  for (int hl = w; hl < nhl; hl += NW) {
+    const float* qp = a.q + ((size_t)r * a.nh + hf + hl) * HD + lane;
     float x[KS];
     float amax = 0.0f;
 #pragma unroll
-    for (int kk = 0; kk < KS; kk++) {
-      x[kk] = live ? a.q[((size_t)r * a.nh + h) * HD + 64 * kk + lane] : 0.0f;
-      amax = __builtin_fmaxf(amax, __builtin_fabsf(x[kk]));
-    }
+    for (int kk = 0; kk < KS; kk++) x[kk] = qp[64 * kk];
+    if (u0 < n && hl == w) load(B0, ks0, u0);
+#pragma unroll
+    for (int kk = 0; kk < KS; kk++) amax = __builtin_fmaxf(amax, __builtin_fabsf(x[kk]));
     amax = wave_max(amax);
     const float qinv = amax > 0.0f ? 127.0f / amax : 0.0f;
 #pragma unroll
@@ -504,231 +558,190 @@ __global__ __launch_bounds__(FUSED_T) void attn_fused_kernel(const AttnArgs a) {
     }
     if (lane == 0) qsc[hl] = amax / 127.0f;
   }
-  __syncthreads();
-  v4i A[KS];
+  if (w >= nhl && u0 < n) load(B0, ks0, u0);
+  if (u0 + 16 * NW < n) load(B1, ks1, u0 + 16 * NW);
+
+  // ---- V: wave w takes the 64-dim block w % KS and the 64-slot steps w / KS,
+  // + NSL, ...; lane (c, q4) loads the 16 bytes [4 dims][4 slots] of dims
+  // 4 c .. 4 c + 3 and slot groups 4 q4 + r, r = 0..3: register q of the four
+  // loads is one MFMA B operand (column c = dim 4 c + q).  The first steps do
+  // not depend on the weights: in flight through scores and softmax.
+  const int db = w % KS, sl = w / KS;
+  const int steps = sl < NSL ? G.dom_steps : 0;
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(G.vc, (uint32_t)((size_t)((G.k_len + 3) >> 2) * kvd * 4));
+  auto loadv = [&](v4i* V, int step) {
+    const int gi = (G.dom_slot(step) >> 2) + 4 * q4;
+    const uint32_t at = ((uint32_t)gi * (uint32_t)kvd + (uint32_t)(g * HD + 64 * db + 4 * c16)) * 4u;
 #pragma unroll
-  for (int kk = 0; kk < KS; kk++)
-    A[kk] = *(const v4i*)(qq + (lane & 15) * QROW + 64 * kk + 16 * (lane >> 4));
-  auto tile = [&](const v4i* B, float kscale, int tt) {
-    v4i acc = {0, 0, 0, 0};
-#pragma unroll
-    for (int kk = 0; kk < KS; kk++) acc = mfma16(A[kk], B[kk], acc);
-    const int t = tt + (lane & 15);
-    if (t < G.en) {
-      const int u = t - G.st;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int hl = 4 * (lane >> 4) + i;
-        if (hl < grp) E[(size_t)hl * 16 * S + (u & 15) * S + (u >> 4)] = ((float)acc[i] * qsc[hl]) * kscale;
-      }
-    }
+    for (int rr = 0; rr < 4; rr++) V[rr] = buf_load_b128(rv, at, (uint32_t)(rr * kvd * 4));
   };
-  for (; t0 < G.en; t0 += 32 * NW) {
-    if (t0 + 16 * NW < G.en) load(B1, ks1, t0 + 16 * NW);
-    tile(B0, ks0, t0);
-    if (t0 + 16 * NW >= G.en) break;
-    if (t0 + 32 * NW < G.en) load(B0, ks0, t0 + 32 * NW);
-    tile(B1, ks1, t0 + 16 * NW);
-  }
-  // ---- P.V: wave w takes the 16-dim tiles w, w + NW, ...; every slot step,
-  // three planes, sums in registers
-  const int hl = lane & 15, q4 = lane >> 4;
-  const bool alive = live_head(hl);
-  const int ngroups = (G.k_len + 3) >> 2;
-  const __amdgpu_buffer_rsrc_t rv = make_rsrc(G.vc, (uint32_t)((size_t)ngroups * kvd * 4));
-  constexpr int NTW = (HD / 16 + NW - 1) / NW;  // dim tiles per wave
-  v4i D[3][NTW];
-#pragma unroll
-  for (int p = 0; p < 3; p++)
-#pragma unroll
-    for (int i = 0; i < NTW; i++) D[p][i] = v4i{0, 0, 0, 0};
-  auto loadv = [&](int* B, int step) {
-    const int s0 = G.dom_lo + 64 * step;
-#pragma unroll
-    for (int i = 0; i < NTW; i++) {
-      const int nt = w + NW * i;
-      const uint32_t j = (uint32_t)(g * HD + 16 * nt + hl);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int gi = (s0 >> 2) + 4 * q4 + q;
-        B[4 * i + q] = (nt < HD / 16 && gi < ngroups)
-                           ? buf_load_b32(rv, ((uint32_t)gi * (uint32_t)kvd + j) * 4u, 0)
-                           : 0;
-      }
-    }
-  };
-  // the first two V steps do not depend on the weights: in flight through
-  // the softmax and the plane writes
-  int V0[4 * NTW], V1[4 * NTW];
-  const int steps = G.dom_steps;
-  if (steps > 0) loadv(V0, 0);
-  if (steps > 1) loadv(V1, 1);
+  v4i V0[4], V1[4];
+  if (sl < steps) loadv(V0, sl);
   __syncthreads();
 
-  // ---- softmax: wave hl owns head hl; the maximum and the exponentials
-  float* Eh = E + (size_t)w * 16 * S;
-  const bool mine = w < grp && live_head(w);
+  // ---- scores; each head's maximum is taken on the way to LDS
+  float hmax[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  {
+    float qs4[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) qs4[i] = qsc[4 * q4 + i];
+    auto tile = [&](const v4i* B, int ksc, int ut) {
+      v4i acc = {0, 0, 0, 0};
+#pragma unroll
+      for (int kk = 0; kk < KS; kk++)
+        acc = mfma16(*(const v4i*)(qq + c16 * QROW + 64 * kk + 16 * q4), B[kk], acc);
+      const int u = ut + c16;
+      const float kscale = __int_as_float(ksc);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int hl = 4 * q4 + i;
+        if (u < n && hl < nhl) {
+          const float s = ((float)acc[i] * qs4[i]) * kscale;
+          hmax[i] = __builtin_fmaxf(hmax[i], s);
+          E[(size_t)hl * 16 * S + (u & 15) * S + (u >> 4)] = s;
+        }
+      }
+    };
+#pragma unroll 1
+    for (; u0 < n; u0 += 32 * NW) {
+      tile(B0, ks0, u0);
+      if (u0 + 16 * NW >= n) break;
+      if (u0 + 32 * NW < n) load(B0, ks0, u0 + 32 * NW);
+      tile(B1, ks1, u0 + 16 * NW);
+      if (u0 + 48 * NW < n) load(B1, ks1, u0 + 48 * NW);
+    }
+  }
+  if (sl + NSL < steps) loadv(V1, sl + NSL);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float m = row16_max(hmax[i]);
+    if (c16 == 0 && 4 * q4 + i < nhl) smax[16 * (4 * q4 + i) + w] = m;
+  }
+
+  // ---- softmax: WPH waves per head, one slot (position) per lane
+  const int WPH = NW / hpw, hw = w / WPH, sub = w - hw * WPH, first = 64 * sub + lane;
+  const bool mine = hw < nhl && hf + hw >= hb && hf + hw < he;
+  float* Eh = E + (size_t)hw * 16 * S;
+  const __amdgpu_buffer_rsrc_t rvs = make_rsrc(G.vs, (uint32_t)G.k_len * 4u);
+  // the first position's V scale is in flight through the exponentials
+  const int vs0 = buf_load_b32(rvs, first < n ? 4u * (uint32_t)G.slot_of(first) : FGM_OOB, 0);
+  __syncthreads();
   if (mine) {
-    float mx = -INFINITY;
-    for (int u = lane; u < n; u += 64) mx = __builtin_fmaxf(mx, Eh[(u & 15) * S + (u >> 4)]);
-    mx = wave_max(mx);
-    for (int u = lane; u < n; u += 64) {
+    const float mx = row16_max(c16 < NW ? smax[16 * hw + c16] : -INFINITY);
+#pragma unroll 1
+    for (int u = first; u < n; u += 64 * WPH) {
       float* p = Eh + (u & 15) * S + (u >> 4);
       const float x = *p - mx;
       *p = u < n16 ? exp16(x) : (float)exp((double)x);
     }
   }
   __syncthreads();
-  // the reference's sum: lanes 0..15 of the head's wave, chunk order, then
-  // GCC's reduce tree and the tail in order
-  if (mine && lane < 16) {
-    const int nt = n16 >> 4;
-    const float* c = Eh + lane * S;
-    float acc = 0.0f;
-    float4 P[4], Q[4];
-    auto rd = [&](float4* p, int q0) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) p[q] = *(const float4*)(c + q0 + 4 * q);
-    };
-    auto add = [&](const float4* p) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        acc = acc + p[q].x;
-        acc = acc + p[q].y;
-        acc = acc + p[q].z;
-        acc = acc + p[q].w;
-      }
-    };
-    int t = 0;
-    rd(P, 0);
-    for (; t + 32 <= nt; t += 32) {
-      rd(Q, t + 16);
-      __builtin_amdgcn_sched_barrier(0);
-      add(P);
-      __builtin_amdgcn_sched_barrier(0);
-      rd(P, t + 32);
-      __builtin_amdgcn_sched_barrier(0);
-      add(Q);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (t + 16 <= nt) {
-      add(P);
-      t += 16;
-    }
-    for (; t < nt; t++) acc = acc + c[t];
-    acc = acc + row_ror<8>(acc);
-    acc = acc + row_ror<4>(acc);
-    acc = acc + row_ror<2>(acc);
-    float sum = acc + row_ror<1>(acc);
-    if (lane == 0) {
-      for (int u = n16; u < n; u++) sum += Eh[(u & 15) * S + (u >> 4)];
-      winv[w] = 1.0f / sum;
-    }
-  }
-  __syncthreads();
-  // weights (e * inv) * vs in place, and their maximum
+  float wm = 0.0f, inv = 0.0f;
   if (mine) {
-    const float inv = winv[w];
-    float wm = 0.0f;
-    for (int u = lane; u < n; u += 64) {
-      const int t = G.st + u;
-      float* p = Eh + (u & 15) * S + (u >> 4);
-      const float wt = (*p * inv) * G.vs[G.ring ? t % G.ring : t];
-      *p = wt;
-      wm = __builtin_fmaxf(wm, wt);
+    // every wave of the head makes the reference's sum: lanes 0..15 in chunk
+    // order, GCC's reduce tree, the tail in order
+    float sum = 0.0f;
+    if (lane < 16) sum = chunk_sum16(Eh + lane * S, n16 >> 4);
+    sum = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(sum)));
+#pragma unroll 1
+    for (int u = n16; u < n; u++) sum += Eh[(u & 15) * S + (u >> 4)];
+    inv = 1.0f / sum;
+    int vs = vs0;
+#pragma unroll 1
+    for (int u = first; u < n; u += 64 * WPH) {
+      wm = __builtin_fmaxf(wm, (Eh[(u & 15) * S + (u >> 4)] * inv) * __int_as_float(vs));
+      if (u + 64 * WPH < n) vs = buf_load_b32(rvs, 4u * (uint32_t)G.slot_of(u + 64 * WPH), 0);
     }
     wm = wave_max(wm);
-    if (lane == 0) {
-      wqs[w] = wm > 0.0f ? wm / 65535.0f : 0.0f;
-      winv[w] = wm > 0.0f ? 65535.0f / wm : 0.0f;
+    if (lane == 0) wred[w] = wm;
+  }
+  // the planes of the slots that hold no position are zero
+  for (int i = tid; i < G.dom_steps * 4 * 3 * hpw; i += 64 * NW) ((v4i*)PL)[i] = v4i{0, 0, 0, 0};
+  __syncthreads();
+
+  // ---- weight planes by slot
+  if (mine) {
+    wm = row16_max(c16 < WPH ? wred[hw * WPH + c16] : 0.0f);
+    const bool pos = wm > 0.0f;
+    const float wq_inv = 65535.0f / wm;
+    if (sub == 0 && lane == 0) wqs[hw] = pos ? wm / 65535.0f : 0.0f;
+    int vs = vs0;
+#pragma unroll 1
+    for (int u = first; pos && u < n; u += 64 * WPH) {
+      const float wt = (Eh[(u & 15) * S + (u >> 4)] * inv) * __int_as_float(vs);
+      int q = (int)__builtin_fmaf(wt, wq_inv, 0.5f);
+      q = q > 65535 ? 65535 : (q < 0 ? 0 : q);
+      const int s = G.slot_of(u), d = G.dom_off(s);
+      q <<= G.twice(s) ? 1 : 0;
+      int8_t* p = PL + (size_t)(d >> 4) * (48 * hpw) + hw * 16 + (d & 15);
+      p[0] = (int8_t)(q >> 14);
+      p[16 * hpw] = (int8_t)((q >> 7) & 127);
+      p[32 * hpw] = (int8_t)(q & 127);
+      if (u + 64 * WPH < n) vs = buf_load_b32(rvs, 4u * (uint32_t)G.slot_of(u + 64 * WPH), 0);
     }
   }
   __syncthreads();
 
-  // ---- weight planes by slot, every head, four slots per thread
-  const int dom_hi = G.dom_lo + 64 * G.dom_steps;
-  for (int s4 = G.dom_lo + 4 * tid; s4 < dom_hi; s4 += 4 * FUSED_T) {
-    int tt[4];
-    int mult[4];
+  // ---- P.V: the A operand's rows are (plane, head), 3 hpw of them in one
+  // operand or two; sums over the wave's steps in registers
+  v4i D0[4], D1[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int s = s4 + e;
-      mult[e] = (s >= G.lo0 && s < G.hi0) + (G.nrun == 2 && s >= G.lo1 && s < G.hi1);
-      int t;
-      bool ok;
-      if (!G.ring) {
-        t = s, ok = s >= G.st && s < G.en;
-      } else {
-        const int d = ((G.en - 1 - s) % G.ring + G.ring) % G.ring;
-        t = G.en - 1 - d, ok = s < G.ring && t >= G.st;
-      }
-      tt[e] = (ok && mult[e]) ? t - G.st : -1;
-    }
-    int8_t* pb = PL + (size_t)((s4 - G.dom_lo) >> 4) * (48 * grp) + (s4 & 15);
-    for (int hl = 0; hl < grp; hl++) {
-      const float* Ehl = E + (size_t)hl * 16 * S;
-      const bool pos = live_head(hl) && wqs[hl] > 0.0f;
-      uint32_t pa = 0, pbb = 0, pc = 0;
+  for (int q = 0; q < 4; q++) D0[q] = D1[q] = v4i{0, 0, 0, 0};
+  const bool two = 3 * hpw > 16;
+  auto mulv = [&](const v4i* V, int step) {
+    const int8_t* wp = PL + (size_t)(4 * step + q4) * (48 * hpw) + c16 * 16;
+    const v4i A0 = *(const v4i*)wp;
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        int W = 0;
-        if (pos && tt[e] >= 0) {
-          const int u = tt[e];
-          int q = (int)__builtin_fmaf(Ehl[(u & 15) * S + (u >> 4)], winv[hl], 0.5f);
-          q = q > 65535 ? 65535 : (q < 0 ? 0 : q);
-          W = mult[e] * q;
-        }
-        pa |= (uint32_t)(W >> 14) << (8 * e);
-        pbb |= (uint32_t)((W >> 7) & 127) << (8 * e);
-        pc |= (uint32_t)(W & 127) << (8 * e);
-      }
-      *(uint32_t*)(pb + hl * 16) = pa;
-      *(uint32_t*)(pb + 16 * grp + hl * 16) = pbb;
-      *(uint32_t*)(pb + 32 * grp + hl * 16) = pc;
-    }
-  }
-  __syncthreads();
-
-  auto mulv = [&](const int* B, int step) {
-    const int8_t* wp = PL + (size_t)(4 * step + q4) * (48 * grp) + hl * 16;
-    v4i Ap[3];
+    for (int q = 0; q < 4; q++) D0[q] = mfma16(A0, v4i{V[0][q], V[1][q], V[2][q], V[3][q]}, D0[q]);
+    if (two) {
+      const v4i A1 = *(const v4i*)(wp + 256);
 #pragma unroll
-    for (int p = 0; p < 3; p++) Ap[p] = alive ? *(const v4i*)(wp + p * 16 * grp) : v4i{0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < NTW; i++) {
-      const v4i b = {B[4 * i], B[4 * i + 1], B[4 * i + 2], B[4 * i + 3]};
-#pragma unroll
-      for (int p = 0; p < 3; p++) D[p][i] = mfma16(Ap[p], b, D[p][i]);
+      for (int q = 0; q < 4; q++) D1[q] = mfma16(A1, v4i{V[0][q], V[1][q], V[2][q], V[3][q]}, D1[q]);
     }
   };
-  for (int st = 0; st < steps; st += 2) {
+#pragma unroll 1
+  for (int st = sl; st < steps; st += 2 * NSL) {
     mulv(V0, st);
-    if (st + 2 < steps) loadv(V0, st + 2);
-    if (st + 1 >= steps) break;
-    mulv(V1, st + 1);
-    if (st + 3 < steps) loadv(V1, st + 3);
+    if (st + NSL >= steps) break;
+    if (st + 2 * NSL < steps) loadv(V0, st + 2 * NSL);
+    mulv(V1, st + NSL);
+    if (st + 3 * NSL < steps) loadv(V1, st + 3 * NSL);
   }
-  // out = (float)(a 2^14 + b 2^7 + c) * wmax / 65535
+  // the rows' sums to LDS (in the exponentials' place: all read), one
+  // [3 hpw][64] block per wave
+  int32_t* red = (int32_t*)E;
 #pragma unroll
-  for (int i = 0; i < NTW; i++) {
-    const int nt = w + NW * i;
-    if (nt >= HD / 16) continue;
+  for (int i = 0; i < 4; i++) {
+    const int row = 4 * q4 + i;
+    if (row < 3 * hpw) *(v4i*)(red + ((size_t)w * 3 * hpw + row) * 64 + 4 * c16) = v4i{D0[0][i], D0[1][i], D0[2][i], D0[3][i]};
+    if (row + 16 < 3 * hpw)
+      *(v4i*)(red + ((size_t)w * 3 * hpw + row + 16) * 64 + 4 * c16) = v4i{D1[0][i], D1[1][i], D1[2][i], D1[3][i]};
+  }
+  __syncthreads();
+  // sum iw v = a 2^14 + b 2^7 + c (modulo 2^32, as the reference's int32
+  // lanes) over the slices; out = (float)(that) * wmax / 65535
+#pragma unroll 1
+  for (int idx = tid; idx < nhl * HD; idx += 64 * NW) {
+    const int hr = idx / HD, d = idx - hr * HD;
+    uint32_t t = 0;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int hr = 4 * (lane >> 4) + k, h = g * grp + hr;
-      if (!live_head(hr)) continue;
-      const uint32_t tot = ((uint32_t)D[0][i][k] << 14) + ((uint32_t)D[1][i][k] << 7) + (uint32_t)D[2][i][k];
-      a.out[((size_t)r * a.nh + h) * HD + 16 * nt + (lane & 15)] = (float)(int32_t)tot * wqs[hr];
+    for (int s = 0; s < NSL; s++) {
+      const int32_t* p = red + (size_t)(s * KS + (d >> 6)) * 3 * hpw * 64 + hr * 64 + (d & 63);
+      t += ((uint32_t)p[0] << 14) + ((uint32_t)p[64 * hpw] << 7) + (uint32_t)p[128 * hpw];
     }
+    if (hf + hr >= hb && hf + hr < he)
+      a.out[((size_t)r * a.nh + hf + hr) * HD + d] = (float)(int32_t)t * wqs[hr];
   }
 }
 
 template <int KS>
 hipError_t launch_fused(const AttnArgs& a, size_t lds, hipStream_t st) {
-  static hipError_t attr = hipFuncSetAttribute((const void*)attn_fused_kernel<KS>,
+  constexpr int NW = fused_waves(64 * KS);
+  static hipError_t attr = hipFuncSetAttribute((const void*)attn_fused_kernel<KS, NW>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(attn_fused_kernel<KS>, dim3(a.m * a.kvh), dim3(FUSED_T), lds, st, a);
+  const int hs = (a.nh / a.kvh + a.hpw - 1) / a.hpw;
+  hipLaunchKernelGGL((attn_fused_kernel<KS, NW>), dim3(a.m * a.kvh * hs), dim3(64 * NW), lds, st, a);
   return hipGetLastError();
 }
 
@@ -821,24 +834,30 @@ size_t fgm_attn_layout(AttnArgs* a, void* base, int m, int nh, int kvh, int hd, 
   return off;
 }
 
-hipError_t fgm_launch_attn(const AttnArgs& a, int max_n, hipStream_t st) {
+hipError_t fgm_launch_attn(const AttnArgs& a, hipStream_t st) {
+  const int max_n = a.max_n;
   if (a.m <= 0 || a.h1 <= a.h0) return hipSuccess;
   hipError_t e = hipSuccess;
   // one launch when every row is short and a kv group fits the workgroup;
   // FGM_ATTN_FUSED=0 keeps the four-launch path (for comparison and tests)
   const int grp = a.nh / a.kvh;
   const char* fz = getenv("FGM_ATTN_FUSED");
-  const size_t flds = fused_lds(a.hd, grp, max_n, a.wpl_blocks);
-  if (max_n <= FUSED_MAX_N && grp <= FUSED_MAX_GRP && !(fz && fz[0] == '0') && flds <= 160 * 1024) {
+  // query heads per workgroup: as few as fill the chip (256 CUs) once
+  AttnArgs f = a;
+  f.hpw = 1;
+  while (f.hpw < grp && a.m * a.kvh * ((grp + f.hpw - 1) / f.hpw) > 256) f.hpw *= 2;
+  f.hpw = std::min(f.hpw, grp);
+  const size_t flds = fused_lds(fused_waves(a.hd), a.hd, f.hpw, a.max_n, a.max_steps);
+  if (a.max_n <= FUSED_MAX_N && grp <= FUSED_MAX_GRP && !(fz && fz[0] == '0') && flds <= 160 * 1024) {
     switch (a.hd / 64) {
-      case 1: return launch_fused<1>(a, flds, st);
-      case 2: return launch_fused<2>(a, flds, st);
-      case 3: return launch_fused<3>(a, flds, st);
-      case 4: return launch_fused<4>(a, flds, st);
-      case 5: return launch_fused<5>(a, flds, st);
-      case 6: return launch_fused<6>(a, flds, st);
-      case 7: return launch_fused<7>(a, flds, st);
-      case 8: return launch_fused<8>(a, flds, st);
+      case 1: return launch_fused<1>(f, flds, st);
+      case 2: return launch_fused<2>(f, flds, st);
+      case 3: return launch_fused<3>(f, flds, st);
+      case 4: return launch_fused<4>(f, flds, st);
+      case 5: return launch_fused<5>(f, flds, st);
+      case 6: return launch_fused<6>(f, flds, st);
+      case 7: return launch_fused<7>(f, flds, st);
+      case 8: return launch_fused<8>(f, flds, st);
       default: return hipErrorInvalidValue;
     }
   }

@@ -125,10 +125,15 @@ struct AttnSeq {
   const int8_t* vc;   // transposed, [ceil(k_len / 4)][kv_heads * head_dim][4]
   const float* vs;    // [k_len]
   int k_len, ring, pos0, lo, nrows, row0;
+  int st0, slot0;     // start of the first row's range and its slot
 };
 struct AttnArgs {
   AttnSeq seq[FGM_ATTN_MAX_SEQ];
+  int row0[FGM_ATTN_MAX_SEQ];  // seq[i].row0, INT_MAX past nseq (ascending: row r is in the last i with row0[i] <= r)
   int nseq, m, nh, kvh, hd, window, h0, h1;
+  int one_row;           // every sequence has exactly one row
+  int max_n, max_steps;  // over the rows: positions, P.V slot steps
+  int hpw;               // query heads per workgroup (single-launch path)
   float* out;
   const float* q;
   // scratch
@@ -144,34 +149,45 @@ struct AttnArgs {
   int p3_chunks;      // P.V slot chunks (4 * p3_spw steps) per (row, kv head)
 };
 // A row's attended range and the reference's slot runs (ops.c:560-572) as
-// four-slot-aligned spans [lo, hi); the P.V slot domain is
-// [dom_lo, dom_lo + 64 dom_steps).  Shared by the host (grid sizing) and the
-// kernels.
+// four-slot-aligned spans: [lo0, hi0), and [0, hi1) when the range wraps in
+// its ring (hi1 = 0 otherwise; the two spans then share at most the group of
+// slot s0, which the reference counts twice).  The P.V product walks the
+// 64-slot steps that the spans touch: step i covers the slots from
+// dom_lo + 64 i, plus `gap` from step nst1 on (the unused middle of a wrapped
+// ring).  Shared by the host (grid sizing) and the kernels.
 struct AttnSpan {
-  int st, en, n, nrun, lo0, hi0, lo1, hi1, dom_lo, dom_steps;
+  int st, en, n, s0, lo0, hi0, hi1, dom_lo, dom_steps, nst1, gap;
 };
-__host__ __device__ inline AttnSpan attn_span(int en, int lo, int window, int ring) {
+template <class F>  // slot_of_start(st): st % ring
+__host__ __device__ inline AttnSpan attn_span(int en, int lo, int window, int ring, F slot_of_start) {
   AttnSpan g;
   g.en = en;
   g.st = window > 0 ? (en - window > 0 ? en - window : 0) : lo;
   g.n = g.en - g.st;
-  g.lo1 = g.hi1 = 0;
-  if (!ring) {
-    g.lo0 = g.st, g.hi0 = g.en, g.nrun = 1;
-  } else if (g.n >= ring) {
-    g.lo0 = 0, g.hi0 = ring, g.nrun = 1;
+  g.s0 = slot_of_start(g.st);
+  g.lo0 = g.s0 & ~3, g.hi1 = 0;
+  if (ring && g.n >= ring) {  // one run over the whole ring
+    g.lo0 = 0;
+    g.hi0 = (ring + 3) & ~3;
+  } else if (ring && g.s0 + g.n > ring) {
+    g.hi0 = (ring + 3) & ~3;
+    g.hi1 = (g.s0 + g.n - ring + 3) & ~3;
   } else {
-    const int s0 = g.st % ring;
-    if (s0 + g.n <= ring) {
-      g.lo0 = s0, g.hi0 = s0 + g.n, g.nrun = 1;
-    } else {
-      g.lo0 = s0, g.hi0 = ring, g.lo1 = 0, g.hi1 = s0 + g.n - ring, g.nrun = 2;
-    }
+    g.hi0 = (g.s0 + g.n + 3) & ~3;
   }
-  g.lo0 &= ~3, g.hi0 = (g.hi0 + 3) & ~3;
-  g.lo1 &= ~3, g.hi1 = (g.hi1 + 3) & ~3;
-  g.dom_lo = (g.nrun == 2 ? 0 : g.lo0) & ~63;
-  g.dom_steps = (g.hi0 - g.dom_lo + 63) >> 6;
+  g.nst1 = (g.hi1 + 63) >> 6, g.gap = 0;
+  const int base0 = g.lo0 & ~63;
+  if (g.hi1 == 0) {
+    g.dom_lo = base0;
+    g.dom_steps = (g.hi0 - base0 + 63) >> 6;
+  } else if (base0 > 64 * g.nst1) {
+    g.dom_lo = 0;
+    g.gap = base0 - 64 * g.nst1;
+    g.dom_steps = g.nst1 + ((g.hi0 - base0 + 63) >> 6);
+  } else {
+    g.dom_lo = 0;
+    g.dom_steps = (g.hi0 + 63) >> 6;
+  }
   return g;
 }
 // P.V slot chunks per (row, kv head): enough workgroups to fill the chip
@@ -184,7 +200,7 @@ inline int attn_pv_chunks(int m, int kvh, int hd) {
 // of the ring size) are at most max_span; returns the bytes and fills the
 // scratch pointers of `a` when base != nullptr.
 size_t fgm_attn_layout(AttnArgs* a, void* base, int m, int nh, int kvh, int hd, int max_span);
-hipError_t fgm_launch_attn(const AttnArgs& a, int max_n, hipStream_t st);
+hipError_t fgm_launch_attn(const AttnArgs& a, hipStream_t st);
 // V row scatter into the transposed cache (ops.c:653-657).
 hipError_t fgm_launch_store_v_t(int8_t* vt, const int8_t* src, int n, int slot, hipStream_t st);
 // Quantise m K and V rows (quant_act per row) into one cache at slots

@@ -151,6 +151,32 @@ def test_job_api_batched_decode_and_prefill(attn_path):
     assert exact >= len(want) - 4          # glibc's expf is rarely off by an ulp
 
 
+@pytest.mark.parametrize("nh,kvh,hd,cap,ring,window,pos,rows", [
+    (8, 1, 64, 700, 700, 100, 1440, 3),      # a wrapped range whose ring is mostly unused
+    (8, 1, 64, 701, 699, 5, 1400, 1),        # both spans of the wrap in one slot group
+    (6, 2, 128, 1200, 1200, 1024, 1300, 2),  # the longest single-launch row, three heads per kv head
+    (5, 1, 320, 90, 0, 0, 60, 30),           # five heads, eight waves
+    (8, 1, 64, 64, 64, 33, 500, 32),         # one head per workgroup, the chip just filled
+    (8, 1, 64, 128, 128, 33, 500, 65),       # four heads per workgroup
+    (8, 1, 64, 400, 400, 33, 1000, 260),     # every head in one workgroup
+    (3, 1, 64, 140, 140, 20, 700, 120),      # two of three heads, then the third
+])
+def test_job_heads_split_and_wrapped_rings(nh, kvh, hd, cap, ring, window, pos, rows, attn_path):
+    """The head split by row count and the walk over a wrapped ring's two spans."""
+    t = H.torch()
+    print(f"attn rows {rows} heads {nh} hd {hd} ring {ring} ({attn_path})", flush=True)
+    q, kv = cases.attn_inputs(f"split{rows}", nh, kvh, hd, cap, 1.0)
+    qrows = np.stack([np.roll(q, 17 * r) for r in range(rows)])
+    out = t.full((rows * nh * hd,), 7.0, dtype=t.float32, device="cuda")
+    K.attend(out, H.dev(qrows.reshape(-1)), [(*dev_kv(kv), cap, ring, pos, rows)], nh, kvh, hd, window)
+    got = H.host(out).reshape(rows, nh * hd)
+    for r in range(rows):
+        en = pos + r + 1
+        st = max(en - window, 0) if window else 0
+        want, noncr = oracle_out("heads", qrows[r], kv, nh, st, en, 0, nh, ring, 0.0)
+        same_or_tail_close(got[r], want, noncr)
+
+
 def test_kv_store_matches_reference_write_path():
     """fgm_hip_kv_store_dev equals quant_act + store_v_t per row (the forward
     pass's write, forward.rs:515-548), linear and wrapping ring."""
