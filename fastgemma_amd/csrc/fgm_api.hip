@@ -1050,9 +1050,12 @@ static int attn_plan(AttnArgs& a, int* max_span) {
   if (a.nseq < 0 || a.nseq > FGM_ATTN_MAX_SEQ)
     return fail(FGM_HIP_EINVAL, "attend: %d sequences (at most %d per call)", a.nseq, FGM_ATTN_MAX_SEQ);
   if (!a.out || !a.q) return fail(FGM_HIP_EINVAL, "attend: out or q is NULL");
-  int m = 0, mn = 0, ms = 1, p1max = 1, steps_max = 1;
-  long long tiles = 0;
+  const int grp = a.nh / a.kvh;
+  int m = 0, mn = 0, ms = 1, steps_max = 1;
   std::fill(a.row0, a.row0 + FGM_ATTN_MAX_SEQ, INT_MAX);
+  std::fill(a.tile0, a.tile0 + FGM_ATTN_MAX_SEQ, INT_MAX);
+  a.one_row = 1;
+  a.dup = 0;
   for (int i = 0; i < a.nseq; i++) {
     AttnSeq& s = a.seq[i];
     if (s.nrows < 0) return fail(FGM_HIP_EINVAL, "attend: sequence %d has %d rows", i, s.nrows);
@@ -1062,40 +1065,56 @@ static int attn_plan(AttnArgs& a, int* max_span) {
       return fail(FGM_HIP_EINVAL, "attend: sequence %d: k_len=%d ring=%d", i, s.k_len, s.ring);
     s.row0 = a.row0[i] = m;
     m += s.nrows;
+    a.one_row &= s.nrows == 1;
     for (int j = 0; j < s.nrows; j++) {
-      const AttnSpan sp = attn_span(s.pos0 + j + 1, s.lo, a.window, s.ring,
-                                    [&](int st) { return s.ring ? st % s.ring : st; });
-      if (j == 0) s.st0 = sp.st, s.slot0 = sp.s0;
-      if (sp.st < 0 || sp.n < 0)
-        return fail(FGM_HIP_EINVAL, "attend: sequence %d row %d: range [%d,%d)", i, j, sp.st, sp.en);
-      if (!s.ring && sp.en > s.k_len)
+      const int en = s.pos0 + j + 1, st = attn_start(en, s.lo, a.window), n = en - st;
+      if (st < 0 || n < 0)
+        return fail(FGM_HIP_EINVAL, "attend: sequence %d row %d: range [%d,%d)", i, j, st, en);
+      if (!s.ring && en > s.k_len)
         return fail(FGM_HIP_EINVAL, "attend: sequence %d row %d: position %d outside a cache of %d",
-                    i, j, sp.en - 1, s.k_len);
-      if (s.ring && sp.n > s.ring)
+                    i, j, en - 1, s.k_len);
+      if (s.ring && n > s.ring)
         return fail(FGM_HIP_EINVAL, "attend: sequence %d row %d: %d positions exceed the ring of %d",
-                    i, j, sp.n, s.ring);
-      if (sp.n > FGM_ATTN_MAX_SPAN)
-        return fail(FGM_HIP_EINVAL, "attend: %d positions in one row (at most %d)", sp.n, FGM_ATTN_MAX_SPAN);
-      mn = std::max(mn, sp.n);
-      ms = std::max(ms, std::max(sp.n, s.ring));
-      tiles += (sp.n + 15) / 16;
+                    i, j, n, s.ring);
+      if (n > FGM_ATTN_MAX_SPAN)
+        return fail(FGM_HIP_EINVAL, "attend: %d positions in one row (at most %d)", n, FGM_ATTN_MAX_SPAN);
+      const AttnSpan sp = attn_span(st, en, s.ring, s.ring ? st % s.ring : st);
+      if (j == 0) s.st0 = sp.st, s.slot0 = sp.s0;
+      mn = std::max(mn, n);
+      ms = std::max(ms, std::max(n, s.ring));
       steps_max = std::max(steps_max, sp.dom_steps);
+      a.dup |= sp.lo0 < sp.hi1;
     }
   }
-  // positions per score workgroup: two 16-position tiles per wave while the
-  // launch is small (about 512 workgroups), more once it has thousands
-  const int tpw = (int)std::min<long long>(16, std::max<long long>(2, tiles / (4 * 512)));
-  a.p1_chunk = 64 * tpw;
-  p1max = std::max(1, (mn + a.p1_chunk - 1) / a.p1_chunk);
   a.m = m;
-  a.p1_chunks = p1max;
-  // P.V: the row's 64-slot steps split into at most attn_pv_chunks chunks
-  const int chunks = m ? attn_pv_chunks(m, a.kvh, a.hd) : 1;
-  a.p3_spw = std::max(1, (steps_max + 4 * chunks - 1) / (4 * chunks));
-  a.one_row = 1;
-  for (int i = 0; i < a.nseq; i++) a.one_row &= a.seq[i].nrows == 1;
   a.max_n = mn;
   a.max_steps = steps_max;
+  // Row tiles where the sequences have several rows to share K and V between
+  // (four on average), else every row by itself.
+  a.rt = m >= 4 * a.nseq ? std::max(1, FGM_ATTN_TILE / grp) : 1;
+  a.ntiles = 0;
+  a.tile_steps = 1;
+  for (int i = 0; i < a.nseq; i++) {
+    AttnSeq& s = a.seq[i];
+    a.tile0[i] = a.ntiles;
+    a.ntiles += (s.nrows + a.rt - 1) / a.rt;
+    for (int j = 0; j < s.nrows; j += a.rt) {
+      const int st = attn_start(s.pos0 + j + 1, s.lo, a.window), en = s.pos0 + std::min(j + a.rt, s.nrows);
+      a.tile_steps = std::max(a.tile_steps, attn_span(st, en, s.ring, s.ring ? st % s.ring : st).dom_steps);
+    }
+  }
+  // 64-slot steps per score workgroup: about 512 workgroups
+  const long long units = std::max(1, a.ntiles * a.kvh);
+  a.p1_steps = (int)std::max<long long>(1, std::min<long long>(8, (a.tile_steps * units + 511) / 512));
+  // P.V: one chunk when the tiles and dims fill the chip, else as many as do
+  // (and as the scratch holds)
+  const int dim_wgs = a.rt > 1 ? (a.hd + 255) / 256 : a.hd / 32;
+  const int want = a.rt > 1 ? 256 : 128;
+  int chunks = (int)((want + units * dim_wgs - 1) / (units * dim_wgs));
+  if (m) chunks = std::min(chunks, attn_part_rows(m) / m);
+  chunks = std::max(1, std::min(chunks, a.tile_steps));
+  a.p3_steps = (a.tile_steps + chunks - 1) / chunks;
+  a.p3_chunks = (a.tile_steps + a.p3_steps - 1) / a.p3_steps;
   *max_span = ms;
   return FGM_HIP_OK;
 }
@@ -1109,6 +1128,8 @@ static int attn_run(AttnArgs& a, void* scratch, size_t scratch_bytes, hipStream_
     return fail(FGM_HIP_EINVAL, "attend: scratch of %zu bytes, this call needs %zu", scratch_bytes, need);
   if (((uintptr_t)scratch) & 255) return fail(FGM_HIP_EINVAL, "attend: scratch must be 256-byte aligned");
   fgm_attn_layout(&a, scratch, a.m, a.nh, a.kvh, a.hd, max_span);
+  if (a.tile_steps > a.cap)
+    return fail(FGM_HIP_EINVAL, "attend: a slot domain of %d steps exceeds the scratch's %d", a.tile_steps, a.cap);
   hipError_t e = fgm_launch_attn(a, st);
   return e == hipSuccess ? FGM_HIP_OK : hip_fail(e, "attention launch");
 }

@@ -2,27 +2,35 @@
 // fgm_attend_q8_row (ops.c:353-877), the transposed V store (ops.c:653-657)
 // and the forward pass's KV append (forward.rs:515-548).
 //
-// One call is four launches (one for short rows, see the single-launch path
-// below):
-//  1. attn_scores_kernel: s = ((float)(K.q) * qscale) * kscale for every
-//     (row, head, position).  Each workgroup makes the per-head int8 query
-//     (amax, 127 / amax, round to nearest even, clamp +-127; ops.c:417-433);
-//     K.q is an exact int32 on v_mfma_i32_16x16x64_i8 (heads x positions),
-//     equal to the reference's biased vpdpbusd sum minus its correction.
+// One call is one launch for short rows (see the single-launch path below),
+// else:
+//  1. the scores s = ((float)(K.q) * qscale) * kscale for every (row, head,
+//     slot).  The per-head int8 query (amax, 127 / amax, round to nearest even,
+//     clamp +-127; ops.c:417-433); K.q is an exact int32 on the i8 matrix
+//     instructions, equal to the reference's biased vpdpbusd sum minus its
+//     correction.  Rows by themselves: attn_scores_kernel (heads x slots);
+//     tiles of rows: attn_quant_q_kernel, then attn_scores_tile_kernel.
 //  2. attn_softmax_kernel, one workgroup per (row, head): the maximum, the
 //     exponentials (exp512_ps restated for the 16-wide chunks, a correctly
 //     rounded exp for the n % 16 tail), the reference's summation order (16
 //     lane sums in chunk order, GCC's reduce tree, the tail in order), then
 //     the 16-bit weights iw = (int)fma((e * inv) * vs, 65535 / wmax, 0.5)
-//     clamped to [0, 65535], written by slot as three 7-bit planes
-//     (iw = a 2^14 + b 2^7 + c).  A slot's weight is multiplied by the number
-//     of the reference's four-slot-aligned run spans that contain it, since
-//     ops.c:605-631 walks each span in turn.
-//  3. attn_pv_kernel: sum over slots of iw v, the planes against the
-//     transposed V cache on v_mfma_i32_16x16x64_i8, one exact int32 partial
-//     sum per slot chunk;
-//  4. attn_final_kernel: out = (float)(sum of the partials) * (wmax / 65535)
-//     (integer addition is order-free, so the chunking changes nothing).
+//     clamped to [0, 65535], written by slot as two byte planes.
+//  3. the weighted sum over slots of iw v, against the transposed V cache:
+//     attn_pv_kernel (rows by themselves) or attn_pv_tile_kernel;
+//  4. attn_final_kernel where step 3 left partial sums or a row counts slots
+//     twice: out = (float)(sum) * (wmax / 65535) (integer addition is
+//     order-free, so the chunking changes nothing).
+// Scores, weights and V are walked by cache slot, in the order that they lie
+// in memory; only the softmax maps slots to positions.  Two byte planes hold
+// a 16-bit weight exactly: with the sign bit of both bytes flipped they are
+// the signed digits of iw - 32896 = 256 hi + lo, so
+//   sum iw v = 256 sum hi v + sum lo v + 32896 sum v
+// where the last sum is over every slot of the domain, the same for all rows
+// (a slot outside a row's range has iw = 0), modulo 2^32 as the reference's
+// int32 lanes.  Where a wrapped ring's two four-slot-aligned runs share a
+// group (ops.c:605-631 walks each run's span in turn), its slots count twice:
+// the final step adds them once more.
 // Everything that is not integer arithmetic follows the reference's
 // operation order, so outputs equal its bytes.
 #include <hip/hip_runtime.h>
@@ -68,18 +76,20 @@ FGM_DEV float block_max(float v, float* red) {
   return m;
 }
 
-// One row's view of its sequence: cache, attended range and slot runs.
+// One row's (or row tile's) view of its sequence: cache, attended range (of a
+// tile: the union of its rows') and slot domain.
 struct Geo {
   const int8_t* kc;
   const float* ks;
   const int8_t* vc;
   const float* vs;
-  int k_len, ring, st, en, n;
-  int s0;                           // slot of position st
+  int k_len, ring, n;
+  int s0;                           // slot of the range's first position
   int lo0, hi1;                     // slots [lo0, hi1) lie in both spans (none when lo0 >= hi1)
   int dom_lo, dom_steps, nst1, gap; // slot domain of P.V: see AttnSpan
+  int r0, nr;                       // the tile's rows [r0, r0 + nr)
 
-  __device__ int slot_of(int u) const {  // position st + u, u < n
+  __device__ int slot_of(int u) const {  // position u of the range, u < n
     const int s = s0 + u;
     return ring && s >= ring ? s - ring : s;
   }
@@ -89,43 +99,70 @@ struct Geo {
     const int u = s - s0;
     return u < 0 ? u + ring : u;
   }
-  // offset of slot s in the P.V domain
+  __device__ bool twice(int s) const { return s >= lo0 && s < hi1; }
+  // first slot of a 64-slot step, of a group of four slots of the domain
+  __device__ int dom_slot(int step) const { return dom_lo + 64 * step + (step >= nst1 ? gap : 0); }
+  __device__ int dom_slot4(int qd) const { return dom_lo + 4 * qd + ((qd >> 4) >= nst1 ? gap : 0); }
+  // offset of slot s in the domain
   __device__ int dom_off(int s) const {
     const int d = s - dom_lo;
     return d >= 64 * nst1 + gap ? d - gap : d;
   }
-  __device__ bool twice(int s) const { return s >= lo0 && s < hi1; }
-  __device__ int dom_slot(int step) const { return dom_lo + 64 * step + (step >= nst1 ? gap : 0); }
-  __device__ int dom_slot4(int qd) const { return dom_lo + 4 * qd + ((qd >> 4) >= nst1 ? gap : 0); }
 };
 
-FGM_DEV Geo row_geo(const AttnArgs& a, int r) {
-  // the sequence holding row r: one sequence, or one row each, need no look
-  // at the row table (a dependent fetch of the arguments less); its fields by
-  // that (uniform) index from the kernel argument itself
+typedef const __attribute__((address_space(4))) AttnArgs* KernArgs;
+
+// Index of the sequence that item x (a row or a tile) belongs to.  One
+// sequence, or one row each, need no look at the table (a dependent fetch of
+// the arguments less).
+FGM_DEV int seq_of(const AttnArgs& a, const int* first, int x) {
+  if (a.one_row) return x;
+  if (a.nseq == 1) return 0;
   int i = 0;
-  if (a.one_row) {
-    i = r;
-  } else if (a.nseq > 1) {
 #pragma unroll
-    for (int j = 1; j < FGM_ATTN_MAX_SEQ; j++) i += r >= a.row0[j];
-  }
-  const auto* ka = (const __attribute__((address_space(4))) AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-  const auto& s = ka->seq[__builtin_amdgcn_readfirstlane(i)];
+  for (int j = 1; j < FGM_ATTN_MAX_SEQ; j++) i += x >= first[j];
+  return __builtin_amdgcn_readfirstlane(i);
+}
+
+// The union of the ranges of rows [dr, dr + nr) of sequence i (a uniform
+// index into the kernel argument itself).
+FGM_DEV Geo seq_geo(const AttnArgs& a, int i, int dr, int nr) {
+  const auto& s = ((KernArgs)__builtin_amdgcn_kernarg_segment_ptr())->seq[i];
   Geo g;
   g.kc = s.kc, g.ks = s.ks, g.vc = s.vc, g.vs = s.vs, g.k_len = s.k_len, g.ring = s.ring;
-  const int dr = r - s.row0;
-  const AttnSpan sp = attn_span(s.pos0 + dr + 1, s.lo, a.window, g.ring, [&](int st) {
-    // the slot of the sequence's first row's start is known: no division
-    // unless the rows run past the ring
-    int s0 = s.slot0 + (st - s.st0);
-    if (g.ring && s0 >= g.ring) s0 = s0 < 2 * g.ring ? s0 - g.ring : s0 % g.ring;
-    return s0;
-  });
-  g.st = sp.st, g.en = sp.en, g.n = sp.n, g.s0 = sp.s0;
+  g.r0 = s.row0 + dr, g.nr = nr;
+  const int en = s.pos0 + dr + 1, st = attn_start(en, s.lo, a.window);
+  // the slot of the sequence's first row's start is known: no division
+  // unless the rows run past the ring
+  int s0 = s.slot0 + (st - s.st0);
+  if (g.ring && s0 >= g.ring) s0 = s0 < 2 * g.ring ? s0 - g.ring : s0 % g.ring;
+  const AttnSpan sp = attn_span(st, en + nr - 1, g.ring, s0);
+  g.n = sp.n, g.s0 = s0;
   g.lo0 = sp.lo0, g.hi1 = sp.hi1;
   g.dom_lo = sp.dom_lo, g.dom_steps = sp.dom_steps, g.nst1 = sp.nst1, g.gap = sp.gap;
   return g;
+}
+
+FGM_DEV Geo row_geo(const AttnArgs& a, int r) {
+  const int i = seq_of(a, a.row0, r);
+  return seq_geo(a, i, r - ((KernArgs)__builtin_amdgcn_kernarg_segment_ptr())->seq[i].row0, 1);
+}
+
+FGM_DEV Geo tile_geo(const AttnArgs& a, int t) {
+  const int i = seq_of(a, a.tile0, t);
+  const KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  const int dr = (t - ka->tile0[i]) * a.rt;
+  return seq_geo(a, i, dr, min(a.rt, ka->seq[i].nrows - dr));
+}
+
+// Byte address of the weights of pair (row, head) in its tile: a 64-slot step
+// is [half step of 32 slots][plane hi, lo][pair][32 bytes], so that an MFMA
+// operand of 32 pairs is one contiguous KB.  *plane: bytes from the hi to the
+// lo plane; half steps are 2 planes apart, steps 4.
+FGM_DEV int8_t* planes(const AttnArgs& a, const Geo& T, int r, int g, int hl, int* plane) {
+  const int grp = a.nh / a.kvh;
+  *plane = T.nr * grp * 32;
+  return a.wpl + ((size_t)g * a.m + T.r0) * grp * a.cap * 128 + ((r - T.r0) * grp + hl) * 32;
 }
 
 // The reference's sum of exponentials over the 16-wide chunks, for lanes
@@ -171,9 +208,10 @@ FGM_DEV float chunk_sum16(const float* c, int nt) {
   return acc + row_ror<1>(acc);
 }
 
-// ------------------------------------------------------------- 1. scores
-// grid (p1_chunks, m * kvh), 256 threads; wave w takes the 16-position tiles
-// w, w + 4, ... of the workgroup's chunk.
+// --------------------------------------------------- 1. scores, single rows
+// grid (score chunks, m * kvh), 256 threads; wave w takes the 16-slot tiles
+// w, w + 4, ... of the workgroup's steps.  K is read 64 bytes a row and
+// instruction, the next tile in flight while one multiplies.
 template <int KS>  // head_dim / 64
 __global__ __launch_bounds__(256) void attn_scores_kernel(const AttnArgs a) {
   constexpr int HD = KS * 64, QROW = HD + 16;  // padded LDS row: conflict-free fragment reads
@@ -181,33 +219,31 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(const AttnArgs a) {
   __shared__ float qsc[16];
   const int r = blockIdx.y / a.kvh, g = blockIdx.y - r * a.kvh;
   const Geo G = row_geo(a, r);
-  const int t_beg = G.st + (int)blockIdx.x * a.p1_chunk;
-  if (t_beg >= G.en) return;
+  const int d_beg = (int)blockIdx.x * 64 * a.p1_steps;
+  const int d_end = min(d_beg + 64 * a.p1_steps, 64 * G.dom_steps);
+  if (d_beg >= d_end) return;
   const int grp = a.nh / a.kvh;
   const int hb = max(a.h0, g * grp), he = min(a.h1, (g + 1) * grp);
   if (hb >= he) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lane = threadIdx.x & 63, w = wave_id();
 
   const int kvd = a.kvh * HD;
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(G.kc, (uint32_t)((size_t)G.k_len * kvd));
-  const int t_end = min(t_beg + a.p1_chunk, G.en);
-  float* srow = a.sc + (size_t)r * a.nh * a.sc_stride;
-  // the wave's tiles t0 = t_beg + 16 w + 64 i; a tile's K and K scale are in
-  // flight while the previous tile multiplies (the first while the query is
-  // quantised)
-  auto load = [&](v4i* B, float& kscale, int t0) {
-    const int t = t0 + (lane & 15);
-    const bool ok = t < t_end;
-    const int slot = ok ? G.slot_of(t - G.st) : 0;
-    const uint32_t base = ok ? (uint32_t)slot * (uint32_t)kvd + (uint32_t)(g * HD + 16 * (lane >> 4)) : FGM_OOB;
+  const __amdgpu_buffer_rsrc_t rks = make_rsrc(G.ks, (uint32_t)G.k_len * 4u);
+  float* srow = a.sc + (size_t)r * a.nh * (64 * a.cap);
+  auto load = [&](v4i* B, int& kscale, int d0) {
+    const int slot = G.dom_slot4(d0 >> 2) + (lane & 15);
+    const uint32_t base =
+        slot < G.k_len ? (uint32_t)slot * (uint32_t)kvd + (uint32_t)(g * HD + 16 * (lane >> 4)) : FGM_OOB;
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) B[kk] = buf_load_b128(rk, base, 64 * kk);
-    kscale = ok ? G.ks[slot] : 0.0f;
+    kscale = buf_load_b32(rks, slot < G.k_len ? 4u * (uint32_t)slot : FGM_OOB, 0);
   };
   v4i B0[KS], B1[KS];
-  float ks0 = 0.0f, ks1 = 0.0f;
-  int t0 = t_beg + 16 * w;
-  if (t0 < t_end) load(B0, ks0, t0);
+  int ks0 = 0, ks1 = 0;
+  int d0 = d_beg + 16 * w;
+  if (d0 < d_end) load(B0, ks0, d0);
+  if (d0 + 64 < d_end) load(B1, ks1, d0 + 64);
 
   // per-head int8 query, one wave per head row; rows past the group are zero
   for (int hl = w; hl < 16; hl += 4) {
@@ -236,230 +272,563 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(const AttnArgs a) {
 #pragma unroll
   for (int kk = 0; kk < KS; kk++)
     A[kk] = *(const v4i*)(qq + (lane & 15) * QROW + 64 * kk + 16 * (lane >> 4));
-  auto tile = [&](const v4i* B, float kscale, int t0) {
+  auto tile = [&](const v4i* B, int kscale, int d) {
     v4i acc = {0, 0, 0, 0};
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) acc = mfma16(A[kk], B[kk], acc);
-    // D: lane, register i -> head row 4 (lane / 16) + i, position t
-    const int t = t0 + (lane & 15);
-    if (t < t_end) {
+    // D: lane, register i -> head row 4 (lane / 16) + i, slot lane % 16
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int hl = 4 * (lane >> 4) + i, h = g * grp + hl;
-        if (hl < grp && h >= hb && h < he)
-          srow[(size_t)h * a.sc_stride + (t - G.st)] = ((float)acc[i] * qsc[hl]) * kscale;
-      }
+    for (int i = 0; i < 4; i++) {
+      const int hl = 4 * (lane >> 4) + i, h = g * grp + hl;
+      if (hl < grp && h >= hb && h < he)
+        srow[(size_t)h * (64 * a.cap) + d + (lane & 15)] = ((float)acc[i] * qsc[hl]) * __int_as_float(kscale);
     }
   };
-  for (; t0 < t_end; t0 += 128) {
-    if (t0 + 64 < t_end) load(B1, ks1, t0 + 64);
-    tile(B0, ks0, t0);
-    if (t0 + 64 >= t_end) break;
-    if (t0 + 128 < t_end) load(B0, ks0, t0 + 128);
-    tile(B1, ks1, t0 + 64);
+  for (; d0 < d_end; d0 += 128) {
+    tile(B0, ks0, d0);
+    if (d0 + 64 >= d_end) break;
+    if (d0 + 128 < d_end) load(B0, ks0, d0 + 128);
+    tile(B1, ks1, d0 + 64);
+    if (d0 + 192 < d_end) load(B1, ks1, d0 + 192);
+  }
+}
+
+// ---------------------------------------------------- 1. scores, row tiles
+// The int8 query of every (row, head), one wave each: into the partial sums'
+// place (free until P.V), its scale into wq's (free until the softmax).
+__global__ __launch_bounds__(256) void attn_quant_q_kernel(const float* q, int8_t* q8, float* qsc, int count, int hd) {
+  const int lane = threadIdx.x & 63, i = blockIdx.x * 4 + wave_id();
+  if (i >= count) return;
+  float x[8];
+  float amax = 0.0f;
+#pragma unroll
+  for (int kk = 0; kk < 8; kk++) {
+    x[kk] = 64 * kk < hd ? q[(size_t)i * hd + 64 * kk + lane] : 0.0f;
+    amax = __builtin_fmaxf(amax, __builtin_fabsf(x[kk]));
+  }
+  amax = wave_max(amax);
+  const float qinv = amax > 0.0f ? 127.0f / amax : 0.0f;
+#pragma unroll
+  for (int kk = 0; kk < 8; kk++) {
+    const float v = __builtin_amdgcn_fmed3f(__builtin_rintf(x[kk] * qinv), -127.0f, 127.0f);
+    if (64 * kk < hd) q8[(size_t)i * hd + 64 * kk + lane] = (int8_t)(int)v;
+  }
+  if (lane == 0) qsc[i] = amax / 127.0f;
+}
+
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// grid (score chunks, ntiles * kvh), 256 threads: the 128 (row, head) pairs of
+// a tile x the slots of p1_steps steps on v_mfma_i32_32x32x32_i8, wave w the
+// pairs 32 w ...  A wave keeps its queries (32 x hd bytes) in registers; K
+// goes through LDS in stages of 32 slots, a ring of three filled by 1 KB
+// LDS-DMA units (two stages ahead), so the four waves share each byte of K
+// and a row's K is read once per tile instead of once per row.  LDS rows are
+// hd bytes; their 16-byte chunks are permuted (chunk ^ slot % 8 inside each
+// 128-byte line, by the DMA's source address), so that the fragment reads hit
+// every bank.  Bound by the scores' stores (67 MB at 256 rows x 8 heads x 8192
+// positions, head_dim 512: 129 us with every row reading K for itself, 21 us
+// as tiles, beside 4.5 us for the queries).
+template <int KS>
+__global__ __launch_bounds__(256, 2) void attn_scores_tile_kernel(const AttnArgs a) {
+  constexpr int HD = KS * 64, SWZ = KS % 2 ? 3 : 7;
+  constexpr int UPW = (2 * KS + 3) / 4, STAGE = UPW * 4096, NSTORE = 16;
+  constexpr int MAXP = 8;  // steps per workgroup, at most
+  __shared__ __attribute__((aligned(1024))) int8_t ring[3 * STAGE];
+  __shared__ float ksl[64 * MAXP];
+  const int t = blockIdx.y / a.kvh, g = blockIdx.y - t * a.kvh;
+  const Geo T = tile_geo(a, t);
+  const int step0 = (int)blockIdx.x * a.p1_steps, nsteps = min(a.p1_steps, T.dom_steps - step0);
+  if (nsteps <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+  const int grp = a.nh / a.kvh, pairs = T.nr * grp;
+  const int kvd = a.kvh * HD;
+  const v4i rk = rsrc_words(T.kc, (uint32_t)((size_t)T.k_len * kvd));
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)ring;
+  // DMA unit 4 j + w of a stage: 64 chunks from chunk 64 (4 j + w) of the
+  // stage's LDS image on; the lane's chunk there is chunk p of slot sl
+  uint32_t src[UPW];
+#pragma unroll
+  for (int j = 0; j < UPW; j++) {
+    const int c = 64 * (4 * j + w) + lane, sl = c / (4 * KS), p = c - sl * (4 * KS);
+    src[j] = (uint32_t)sl * (uint32_t)kvd + (uint32_t)(g * HD + 16 * (p ^ (sl & SWZ)));
+    if (sl >= 32) src[j] = FGM_OOB;
+  }
+  const int nst = 2 * nsteps;
+  auto issue = [&](int s) {
+    const uint32_t at = (uint32_t)(T.dom_slot(step0 + (s >> 1)) + 32 * (s & 1)) * (uint32_t)kvd;
+    const uint32_t to = lds0 + (uint32_t)(s % 3) * STAGE + 1024u * w;
+#pragma unroll
+    for (int j = 0; j < UPW; j++) dma16(rk, to + 4096u * j, src[j] == FGM_OOB ? FGM_OOB : src[j] + at, 0);
+  };
+  issue(0);
+  issue(1);
+  // the wave's queries: lane row lane % 32, bytes 32 kk + 16 (lane / 32) ...
+  const int c32 = lane & 31, half = lane >> 5;
+  auto pair_row = [&](int mr) {  // (row, head) index of pair mr of the tile
+    const int rr = mr / grp;
+    return (T.r0 + rr) * a.nh + g * grp + (mr - rr * grp);
+  };
+  const int8_t* q8 = (const int8_t*)a.part;
+  const int mine = min(32 * w + c32, pairs - 1);
+  const int8_t* qp = q8 + (size_t)pair_row(mine) * HD + 16 * half;
+  v4i A[2 * KS];
+#pragma unroll
+  for (int kk = 0; kk < 2 * KS; kk++) A[kk] = *(const v4i*)(qp + 32 * kk);
+  // D: register i of a lane is pair 32 w + 8 (i / 4) + 4 half + i % 4, slot c32
+  float qs[16];
+  int prow[16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int mr = min(32 * w + 8 * (i >> 2) + 4 * half + (i & 3), pairs - 1);
+    prow[i] = pair_row(mr);
+    qs[i] = a.wq[prow[i]];
+  }
+  for (int i = tid; i < 64 * nsteps; i += 256) {
+    const int slot = T.dom_slot4((64 * step0 + i) >> 2) + (i & 3);
+    ksl[i] = slot < T.k_len ? T.ks[slot] : 0.0f;
+  }
+  const bool full = 32 * w + 32 <= pairs, some = 32 * w < pairs;
+  const size_t stride = (size_t)64 * a.cap;
+  // LDS addresses of the four chunk pairs of a 128-byte line
+  int fr[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) fr[j] = c32 * HD + 16 * (((2 * j) ^ half) ^ (c32 & SWZ));
+  wait_vm<0>();
+  for (int s = 0; s < nst; s++) {
+    // Stage s was requested two stages ago; since then the wave has issued
+    // stage s + 1 (UPW loads) and, when all its pairs exist, the 16 stores of
+    // stages s - 2 and s - 1 each.  Stages 0 and 1 are already here.
+    if (s >= 2) {
+      if (!full) wait_vm<0>();
+      else if (s + 1 < nst) wait_vm<2 * NSTORE + UPW>();
+      else wait_vm<2 * NSTORE>();
+    }
+    __syncthreads();
+    if (s + 2 < nst) issue(s + 2);
+    if (!some) continue;
+    const int8_t* img = ring + (s % 3) * STAGE;
+    v16i acc = {};
+#pragma unroll
+    for (int kk = 0; kk < 2 * KS; kk++) {
+      const v4i b = *(const v4i*)(img + fr[kk & 3] + 128 * (kk >> 2));
+      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[kk], b, acc, 0, 0, 0);
+    }
+    const float ksc = ksl[32 * s + c32];
+    float* to = a.sc + 64 * step0 + 32 * s + c32;
+    if (full) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) to[(size_t)prow[i] * stride] = ((float)acc[i] * qs[i]) * ksc;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        if (32 * w + 8 * (i >> 2) + 4 * half + (i & 3) < pairs)
+          to[(size_t)prow[i] * stride] = ((float)acc[i] * qs[i]) * ksc;
+    }
   }
 }
 
 // ---------------------------------------------------- 2. softmax, weights
-// grid (m * (h1 - h0)), T threads; dynamic LDS: the exponentials transposed,
-// e[16 c + j] at lds[j * S + c] (S = 4 mod 64, >= n / 16 + 16), then the
-// reduction slots.
+// grid (m * (h1 - h0)), T threads.  A thread owns NQ groups of four slots,
+// tid + T j, from the load of their scores to the store of their weights: all
+// loads are in flight at once, and only the exponentials go through LDS, for
+// the ordered sum: e[16 c + j] at lds[j * S + c] (S = 4 mod 64, >= n / 16 +
+// 16), then the reduction slots.  A few rows are one dependent chain (8 rows x
+// 8 heads x 8192 positions: 15.2 us walking LDS, 9.5 us from registers); many
+// are bound by VALU issue, about 60 instructions a slot (2048 pairs x 8192:
+// 72 -> 42 us).
 FGM_DEV int exp_stride(int n) { return (((n + 15) >> 4) + 16 + 63) / 64 * 64 + 4; }
 
+template <int NQ>
 __global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
   extern __shared__ float lds[];
   const int nhr = a.h1 - a.h0;
-  const int r = blockIdx.x / nhr, h = a.h0 + ((int)blockIdx.x - r * nhr);
+  // consecutive (row, head) pairs on one XCD: they share lines of the weights
+  int b = blockIdx.x;
+  if ((gridDim.x & 7) == 0) b = (b & 7) * (gridDim.x >> 3) + (b >> 3);
+  const int r = b / nhr, h = a.h0 + (b - r * nhr);
   const int grp = a.nh / a.kvh, g = h / grp, hl = h - g * grp;
-  const Geo G = row_geo(a, r);
-  const int tid = threadIdx.x, T = blockDim.x, nw = T >> 6;
-  const int n = max(G.n, 0), n16 = n & ~15;
-  const int S = exp_stride(n);
+  const int si = seq_of(a, a.row0, r);
+  const KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  const int dr = r - ka->seq[si].row0;
+  const Geo G = seq_geo(a, si, dr, 1);
+  Geo T = G;  // the domain: the row tile's
+  if (a.rt > 1) {
+    const int t0 = dr / a.rt * a.rt;
+    T = seq_geo(a, si, t0, min(a.rt, ka->seq[si].nrows - t0));
+  }
+  const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, nw = nt >> 6, w = wave_id();
+  const int n = max(G.n, 0), n16 = n & ~15, S = exp_stride(n);
   float* red = lds + 16 * S;
-  const float* scr = a.sc + ((size_t)r * a.nh + h) * a.sc_stride;
+  const float* scr = a.sc + ((size_t)r * a.nh + h) * (64 * a.cap);
+  const __amdgpu_buffer_rsrc_t rvs = make_rsrc(G.vs, (uint32_t)G.k_len * 4u);
+  const int nq = 16 * T.dom_steps;
 
-  // raw scores into LDS (eight loads in flight per thread), and their maximum
-  float mx = -INFINITY;
-  for (int b = tid; b < n; b += 8 * T) {
-    float v[8];
+  // A wave's 64 groups j are 256 consecutive domain offsets.  Where all of
+  // them hold positions of the row before its n % 16 tail (`u0` of the first,
+  // the others in order), nothing has to be masked.  Elsewhere, slots outside
+  // the range take part in nothing: their score is -inf, their V scale and so
+  // their weight 0, and their exponential goes to a place that nobody reads.
+  const int DUMP = 16 * S + 24;
+  float e[NQ][4];
+  int vs[NQ][4], u0[NQ];
 #pragma unroll
-    for (int j = 0; j < 8; j++) v[j] = b + j * T < n ? scr[b + j * T] : -INFINITY;
+  for (int j = 0; j < NQ; j++) {
+    const int q0 = 64 * w + nt * j, f = T.dom_slot4(q0), l = T.dom_slot4(q0 + 63) + 3;
+    const int uf = G.pos_of(f), ul = G.pos_of(l);
+    u0[j] = l - f == 255 && q0 + 64 <= nq && uf >= 0 && ul == uf + 255 && ul < n16 ? uf : -1;
+    const int qd = tid + nt * j, s4 = T.dom_slot4(qd);
+    if (u0[j] >= 0) {
+      const float4 v = *(const float4*)(scr + 4 * qd);
+      e[j][0] = v.x, e[j][1] = v.y, e[j][2] = v.z, e[j][3] = v.w;
+      const v4i x = buf_load_b128(rvs, 4u * (uint32_t)s4, 0);
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int u = b + j * T;
-      if (u < n) lds[(u & 15) * S + (u >> 4)] = v[j];
-      mx = __builtin_fmaxf(mx, v[j]);
+      for (int i = 0; i < 4; i++) vs[j][i] = x[i];
+    } else {
+      float4 v = {0, 0, 0, 0};
+      if (qd < nq) v = *(const float4*)(scr + 4 * qd);
+      e[j][0] = v.x, e[j][1] = v.y, e[j][2] = v.z, e[j][3] = v.w;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const bool ok = qd < nq && (unsigned)G.pos_of(s4 + i) < (unsigned)n;
+        vs[j][i] = buf_load_b32(rvs, ok ? 4u * (uint32_t)(s4 + i) : FGM_OOB, 0);
+        e[j][i] = ok ? e[j][i] : -INFINITY;
+      }
     }
   }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < NQ; j++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) mx = __builtin_fmaxf(mx, e[j][i]);
   mx = block_max(mx, red);
-  for (int u = tid; u < n; u += T) {
-    float* p = lds + (u & 15) * S + (u >> 4);
-    const float x = *p - mx;
-    *p = u < n16 ? exp16(x) : (float)exp((double)x);
+  uint64_t tl = 0;  // this thread's slots in the tail
+#pragma unroll
+  for (int j = 0; j < NQ; j++) {
+    if (u0[j] >= 0) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int u = u0[j] + 4 * lane + i;
+        e[j][i] = exp16(e[j][i] - mx);
+        lds[(u & 15) * S + (u >> 4)] = e[j][i];
+      }
+    } else {
+      const int qd = tid + nt * j, s4 = T.dom_slot4(qd);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int u = G.pos_of(s4 + i);
+        const float x = e[j][i] - mx;
+        int at = qd < nq && (unsigned)u < (unsigned)n ? (u & 15) * S + (u >> 4) : DUMP;
+        e[j][i] = exp16(x);
+        // the tail: shifted scores, for lanes 0..15 to exponentiate
+        const bool t = at != DUMP && u >= n16;
+        lds[at] = t ? x : e[j][i];
+        tl |= (uint64_t)t << (4 * j + i);
+      }
+    }
   }
   __syncthreads();
   if (tid < 16) {
+    float t = 0.0f;
+    if (n16 + tid < n) t = (float)exp((double)lds[tid * S + (n16 >> 4)]);
     float sum = chunk_sum16(lds + tid * S, n16 >> 4);
-    if (tid == 0) {
-      for (int u = n16; u < n; u++) sum += lds[(u & 15) * S + (u >> 4)];
-      red[nw] = 1.0f / sum;
-    }
+    for (int u = 0; u < n - n16; u++) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), u));
+    if (n16 + tid < n) lds[tid * S + (n16 >> 4)] = t;
+    if (tid == 0) red[nw] = 1.0f / sum;
   }
   __syncthreads();
   const float inv = red[nw];
-
-  // weights (e * inv) * vs in place of the exponentials, and their maximum
+  if (tl) {
+#pragma unroll
+    for (int j = 0; j < NQ; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (tl >> (4 * j + i) & 1)
+          e[j][i] = lds[(G.pos_of(T.dom_slot4(tid + nt * j) + i) & 15) * S + (n16 >> 4)];
+  }
+  // weights (e * inv) * vs, and their maximum
   float wm = 0.0f;
-  for (int b = tid; b < n; b += 8 * T) {
-    float vsv[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int u = b + j * T;
-      vsv[j] = u < n ? G.vs[G.slot_of(u)] : 0.0f;
-    }
+  for (int j = 0; j < NQ; j++)
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int u = b + j * T;
-      if (u < n) {
-        float* p = lds + (u & 15) * S + (u >> 4);
-        const float wt = (*p * inv) * vsv[j];
-        *p = wt;
-        wm = __builtin_fmaxf(wm, wt);
-      }
+    for (int i = 0; i < 4; i++) {
+      e[j][i] = (e[j][i] * inv) * __int_as_float(vs[j][i]);
+      wm = __builtin_fmaxf(wm, e[j][i]);
     }
-  }
   wm = block_max(wm, red);
-  const bool pos = wm > 0.0f;
-  const float wq_inv = 65535.0f / wm;
-
-  // weight planes for every slot of the P.V domain, four slots per thread
-  int8_t* wp = a.wpl + (size_t)(r * a.kvh + g) * a.wpl_blocks * (48 * grp) + hl * 16;
-  for (int qd = tid; qd < 16 * G.dom_steps; qd += T) {
-    const int s4 = G.dom_slot4(qd);
-    uint32_t pa = 0, pb = 0, pc = 0;
+  const bool some = wm > 0.0f;
+  const float wq_inv = some ? 65535.0f / wm : 0.0f;
+  int plane;
+  int8_t* wp = planes(a, T, r, g, hl, &plane);
+  wp += (size_t)(tid >> 3) * (2 * plane) + 4 * (tid & 7);
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int u = G.pos_of(s4 + e);
-      int W = 0;
-      if (pos && (unsigned)u < (unsigned)n) {
-        int q = (int)__builtin_fmaf(lds[(u & 15) * S + (u >> 4)], wq_inv, 0.5f);
-        q = q > 65535 ? 65535 : (q < 0 ? 0 : q);
-        W = G.twice(s4 + e) ? 2 * q : q;
-      }
-      pa |= (uint32_t)(W >> 14) << (8 * e);
-      pb |= (uint32_t)((W >> 7) & 127) << (8 * e);
-      pc |= (uint32_t)(W & 127) << (8 * e);
-    }
-    int8_t* p = wp + (size_t)(qd >> 2) * (48 * grp) + 4 * (qd & 3);
-    *(uint32_t*)p = pa;
-    *(uint32_t*)(p + 16 * grp) = pb;
-    *(uint32_t*)(p + 32 * grp) = pc;
+  for (int j = 0; j < NQ; j++) {
+    if (tid + nt * j >= nq) continue;
+    uint32_t q[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)  // an empty row's weights are NaN: 0 too
+      q[i] = (uint32_t)min(max((int)__builtin_fmaf(e[j][i], wq_inv, 0.5f), 0), 65535);
+    // the bytes of the four weights, high and low, with flipped sign bits
+    const uint32_t q01 = q[0] | q[1] << 16, q23 = q[2] | q[3] << 16;
+    int8_t* p = wp + (size_t)(nt >> 3) * (2 * plane) * j;
+    *(uint32_t*)p = __builtin_amdgcn_perm(q23, q01, 0x07050301u) ^ 0x80808080u;
+    *(uint32_t*)(p + plane) = __builtin_amdgcn_perm(q23, q01, 0x06040200u) ^ 0x80808080u;
   }
-  if (tid == 0) a.wq[r * a.nh + h] = pos ? wm / 65535.0f : 0.0f;
+  if (tid == 0) a.wq[r * a.nh + h] = some ? wm / 65535.0f : 0.0f;
 }
 
 // ------------------------------------------------------------------ 3. P.V
-// grid (p3_chunks, hd / 64, m * kvh), 256 threads: workgroup (x, y) takes the
-// 64-slot steps [4 spw x, 4 spw (x + 1)) of the row's domain and the dims
-// [64 y, + 64); wave w the steps 4 spw x + 4 s + w, all four 16-dim tiles and
-// all three planes, the next step's operands in flight while one multiplies.
-__global__ __launch_bounds__(256) void attn_pv_kernel(const AttnArgs a) {
-  __shared__ int32_t red[4][16][64];
-  const int r = blockIdx.z / a.kvh, g = blockIdx.z - r * a.kvh;
+constexpr uint32_t IW_BIAS = 32896u;  // 256 * 128 + 128: see the planes above
+
+FGM_DEV int dot4_ones(int x, int c) { return __builtin_amdgcn_sdot4(x, 0x01010101, c, false); }
+
+// Single rows.  grid (hd / 32, m * kvh, p3_chunks), 64 NW threads: workgroup
+// (x, y, z) takes the dims [32 x, + 32) and the steps [p3_steps z, + p3_steps)
+// of the row's domain, wave w the steps w, w + NW, ...; lane (c, q4) loads the
+// 8 bytes [2 dims][4 slots] of dims 2 c, 2 c + 1 and slot groups 4 q4 + r,
+// r = 0..3 (a 128-byte line per group): register q of the four loads is one
+// MFMA B operand (column c = dim 2 c + q).  Four steps are in flight.
+// 8 rows x 8192 slots at head_dim 512: 14.7 us and 4.9 us for the partial
+// sums' launch with 4-byte loads in 2048 workgroups; 13 us so, no partial sums.  The A operand's rows are the heads' hi planes (0..7) and lo
+// planes (8..15), with more than eight heads one operand each.  Sixteen waves
+// so that one workgroup covers all of K where 64 workgroups or more run: the
+// sums stay in the workgroup and need no further launch.
+template <bool TWO>  // more than eight heads
+__global__ __launch_bounds__(TWO ? 512 : 1024) void attn_pv_kernel(const AttnArgs a) {
+  constexpr int NW = TWO ? 8 : 16;
+  __shared__ __attribute__((aligned(16))) int32_t red[NW][17][32];
+  const int r = blockIdx.y / a.kvh, g = blockIdx.y - r * a.kvh;
   const Geo G = row_geo(a, r);
   const int grp = a.nh / a.kvh;
   const int hb = max(a.h0, g * grp), he = min(a.h1, (g + 1) * grp);
   if (hb >= he) return;
-  const int spw = a.p3_spw;
-  const int nchunk = max(1, (G.dom_steps + 4 * spw - 1) / (4 * spw));
-  if ((int)blockIdx.x >= nchunk) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int kvd = a.kvh * a.hd, d0 = 64 * blockIdx.y;
-  const int hl = lane & 15, q4 = lane >> 4;
-  const int h = g * grp + hl;
-  const bool live = hl < grp && h >= hb && h < he;
-  const int ngroups = (G.k_len + 3) >> 2;
-  const __amdgpu_buffer_rsrc_t rv = make_rsrc(G.vc, (uint32_t)((size_t)ngroups * kvd * 4));
-  const int8_t* wrow = a.wpl + (size_t)(r * a.kvh + g) * a.wpl_blocks * (48 * grp) + hl * 16;
-  v4i D[3][4];
+  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+  const int kvd = a.kvh * a.hd, d0 = 32 * blockIdx.x;
+  const int c16 = lane & 15, q4 = lane >> 4;
+  int plane;
+  const int8_t* wp = planes(a, G, r, g, TWO ? c16 : c16 & 7, &plane);
+  wp += (TWO ? 0 : plane * (c16 >> 3)) + (q4 >> 1) * 2 * plane + 16 * (q4 & 1);
+  const bool live = (TWO ? c16 : c16 & 7) < grp;
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(G.vc, (uint32_t)((size_t)((G.k_len + 3) >> 2) * kvd * 4));
+  v4i D0[2], D1[2];
+  int sv[2] = {0, 0};
 #pragma unroll
-  for (int p = 0; p < 3; p++)
+  for (int q = 0; q < 2; q++) D0[q] = D1[q] = v4i{0, 0, 0, 0};
+  auto load = [&](v4i* A, v2i* V, int step) {
+    const uint32_t gi = (uint32_t)(G.dom_slot(step) >> 2) + 4u * q4;
+    const uint32_t at = (gi * (uint32_t)kvd + (uint32_t)(g * a.hd + d0 + 2 * c16)) * 4u;
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) D[p][nt] = v4i{0, 0, 0, 0};
-  // A: plane p, row hl, the 16 slots s0 + 16 q4 + [0, 16); B: dim
-  // d0 + 16 nt + hl, dword q = the four slots of group s0 / 4 + 4 q4 + q
-  auto load = [&](v4i* A, int* B, int step) {
-    const int s0 = G.dom_slot(step);
-    const int8_t* wp = wrow + (size_t)(4 * step + q4) * (48 * grp);
-#pragma unroll
-    for (int p = 0; p < 3; p++) A[p] = live ? *(const v4i*)(wp + p * 16 * grp) : v4i{0, 0, 0, 0};
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const uint32_t j = (uint32_t)(g * a.hd + d0 + 16 * nt + hl);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int gi = (s0 >> 2) + 4 * q4 + q;
-        B[4 * nt + q] = buf_load_b32(rv, gi < ngroups ? ((uint32_t)gi * (uint32_t)kvd + j) * 4u : FGM_OOB, 0);
-      }
+    for (int rr = 0; rr < 4; rr++) V[rr] = buf_load_b64(rv, at + (uint32_t)(rr * kvd * 4), 0);
+    A[0] = A[1] = v4i{0, 0, 0, 0};
+    if (live) {
+      A[0] = *(const v4i*)(wp + (size_t)step * (4 * plane));
+      if constexpr (TWO) A[1] = *(const v4i*)(wp + (size_t)step * (4 * plane) + plane);
     }
   };
-  auto mul = [&](const v4i* A, const int* B) {
+  auto mul = [&](const v4i* A, const v2i* V) {
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const v4i b = {B[4 * nt], B[4 * nt + 1], B[4 * nt + 2], B[4 * nt + 3]};
+    for (int q = 0; q < 2; q++) {
+      const v4i b = {V[0][q], V[1][q], V[2][q], V[3][q]};
+      D0[q] = mfma16(A[0], b, D0[q]);
+      if constexpr (TWO) D1[q] = mfma16(A[1], b, D1[q]);
 #pragma unroll
-      for (int p = 0; p < 3; p++) D[p][nt] = mfma16(A[p], b, D[p][nt]);
+      for (int rr = 0; rr < 4; rr++) sv[q] = dot4_ones(b[rr], sv[q]);
     }
   };
-  const int first = (int)blockIdx.x * 4 * spw;
-  const int last = min(first + 4 * spw, G.dom_steps);
-  v4i A0[3], A1[3];
-  int B0[16], B1[16];
+  const int first = (int)blockIdx.z * a.p3_steps, last = min(first + a.p3_steps, G.dom_steps);
+  v4i A[4][2];
+  v2i V[4][4];
   int step = first + w;
-  if (step < last) load(A0, B0, step);
-  for (; step < last; step += 8) {
-    if (step + 4 < last) load(A1, B1, step + 4);
-    mul(A0, B0);
-    if (step + 4 >= last) break;
-    if (step + 8 < last) load(A0, B0, step + 8);
-    mul(A1, B1);
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (step + NW * i < last) load(A[i], V[i], step + NW * i);
+#pragma unroll 1
+  while (step < last) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      if (step < last) {
+        mul(A[i], V[i]);
+        if (step + 4 * NW < last) load(A[i], V[i], step + 4 * NW);
+      }
+      step += NW;
+    }
   }
-  // sum iw v = a 2^14 + b 2^7 + c (modulo 2^32, as the reference's int32 lanes)
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++)
+  for (int q = 0; q < 2; q++) {
+    sv[q] += __shfl_xor(sv[q], 16, 64);
+    sv[q] += __shfl_xor(sv[q], 32, 64);
+  }
+  // rows 0..15: heads' sums 256 hi (+ lo), or hi and lo of eight; row 16: sum v
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-      red[w][4 * (lane >> 4) + i][16 * nt + (lane & 15)] =
-          (int32_t)(((uint32_t)D[0][nt][i] << 14) + ((uint32_t)D[1][nt][i] << 7) + (uint32_t)D[2][nt][i]);
+  for (int i = 0; i < 4; i++) {
+    const int row = 4 * q4 + i;
+    v2i v;
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+      v[q] = TWO ? (int)(((uint32_t)D0[q][i] << 8) + (uint32_t)D1[q][i])
+                 : (int)(row < 8 ? (uint32_t)D0[q][i] << 8 : (uint32_t)D0[q][i]);
+    *(v2i*)&red[w][row][2 * c16] = v;
+  }
+  if (q4 == 0) *(v2i*)&red[w][16][2 * c16] = v2i{sv[0], sv[1]};
   __syncthreads();
-  int32_t* part = a.part + ((size_t)(r * a.kvh + g) * a.p3_chunks + blockIdx.x) * grp * a.hd + d0;
-  for (int idx = tid; idx < grp * 64; idx += 256) {
-    const int hr = idx >> 6, d = idx & 63;
-    part[(size_t)hr * a.hd + d] = (int32_t)((uint32_t)red[0][hr][d] + (uint32_t)red[1][hr][d] +
-                                            (uint32_t)red[2][hr][d] + (uint32_t)red[3][hr][d]);
+  for (int idx = tid; idx < grp * 32; idx += 64 * NW) {
+    const int hr = idx >> 5, d = idx & 31, h = g * grp + hr;
+    if (h < hb || h >= he) continue;
+    uint32_t t = 0;
+#pragma unroll 4
+    for (int i = 0; i < NW; i++)
+      t += (uint32_t)red[i][hr][d] + (TWO ? 0u : (uint32_t)red[i][8 + hr][d]) + IW_BIAS * (uint32_t)red[i][16][d];
+    const size_t row = (size_t)r * a.nh + h;
+    if (a.p3_chunks == 1 && !a.dup)
+      a.out[row * a.hd + d0 + d] = (float)(int32_t)t * a.wq[row];
+    else
+      a.part[(row * a.p3_chunks + blockIdx.z) * a.hd + d0 + d] = (int32_t)t;
+  }
+}
+
+// Row tiles.  grid (hd / 256 rounded up, ntiles * kvh, p3_chunks), 64 * 4 NG
+// threads (NG = 2, or 1 for head_dim <= 128): the 128 pairs of a tile x 128 NG
+// dims x the chunk's steps on v_mfma_i32_32x32x32_i8.  Wave (mg, ng) takes
+// the pairs 32 mg ... and the dims 128 ng ..., with both planes' sums in
+// registers; its A operands are 16-byte loads of the planes' rows, its B
+// operands 16-byte loads [4 dims][4 slots] of V as above (column c = dim
+// 4 c + q).  The four waves of a dim block read the same V, and the NG waves
+// of a pair block the same planes, out of L1; three half steps are in flight.
+// 256 rows x 8 heads x 8192 slots at head_dim 512: 93 us with every row
+// reading V for itself and three 7-bit planes, 40 us so (54 us while a pair's
+// hi and lo bytes lay side by side, 32-byte pieces of 128-byte lines).
+// sum v: wave mg adds up the half steps mg, mg + 4, ...
+template <int NG>
+__global__ __launch_bounds__(256 * NG, 2) void attn_pv_tile_kernel(const AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) int svl[NG][4][32][4];
+  const int t = blockIdx.y / a.kvh, g = blockIdx.y - t * a.kvh;
+  const Geo T = tile_geo(a, t);
+  const int lane = threadIdx.x & 63, w = wave_id(), mg = w & 3, ng = w >> 2;
+  const int grp = a.nh / a.kvh, pairs = T.nr * grp;
+  const int kvd = a.kvh * a.hd, d0 = (int)blockIdx.x * 128 * NG + 128 * ng;
+  const int c32 = lane & 31, half = lane >> 5;
+  int plane;
+  const int8_t* wp = planes(a, T, T.r0, g, 0, &plane) + min(32 * mg + c32, pairs - 1) * 32 + 16 * half;
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(T.vc, (uint32_t)((size_t)((T.k_len + 3) >> 2) * kvd * 4));
+  v16i H[4], L[4];
+  int sv[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 4; q++) H[q] = L[q] = v16i{};
+  const int first = 2 * (int)blockIdx.z * a.p3_steps, last = min(first + 2 * a.p3_steps, 2 * T.dom_steps);
+  // half steps of 32 slots: V groups 4 half + r of the eight, planes' bytes
+  // 32 hs + 16 half; past the last one, that one again (never multiplied)
+  auto load = [&](v4i* A, v4i* V, int hs) {
+    hs = min(hs, last - 1);
+    const uint32_t gi = (uint32_t)(T.dom_slot(hs >> 1) >> 2) + 8u * (hs & 1) + 4u * half;
+    const uint32_t at = (gi * (uint32_t)kvd + (uint32_t)(g * a.hd + d0 + 4 * c32)) * 4u;
+    const int8_t* p = wp + (size_t)hs * (2 * plane);
+    A[0] = *(const v4i*)p;
+    A[1] = *(const v4i*)(p + plane);
+#pragma unroll
+    for (int rr = 0; rr < 4; rr++) V[rr] = buf_load_b128(rv, at + (uint32_t)(rr * kvd * 4), 0);
+  };
+  auto mul = [&](const v4i* A, const v4i* V, int hs) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const v4i b = {V[0][q], V[1][q], V[2][q], V[3][q]};
+      H[q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], b, H[q], 0, 0, 0);
+      L[q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[1], b, L[q], 0, 0, 0);
+    }
+    if ((hs & 3) == mg) {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int rr = 0; rr < 4; rr++) sv[q] = dot4_ones(V[rr][q], sv[q]);
+    }
+  };
+  if (first < last) {
+    v4i A0[2], A1[2], A2[2], V0[4], V1[4], V2[4];
+    load(A0, V0, first);
+    load(A1, V1, first + 1);
+#pragma unroll 1
+    for (int hs = first; hs < last; hs += 3) {
+      load(A2, V2, hs + 2);
+      mul(A0, V0, hs);
+      if (hs + 1 >= last) break;
+      load(A0, V0, hs + 3);
+      mul(A1, V1, hs + 1);
+      if (hs + 2 >= last) break;
+      load(A1, V1, hs + 4);
+      mul(A2, V2, hs + 2);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) sv[q] += __shfl_xor(sv[q], 32, 64);
+  if (half == 0) *(v4i*)svl[ng][mg][c32] = v4i{sv[0], sv[1], sv[2], sv[3]};
+  __syncthreads();
+  if (d0 + 4 * c32 >= a.hd) return;
+  v4i bias;
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    bias[q] = (int)(IW_BIAS * ((uint32_t)svl[ng][0][c32][q] + (uint32_t)svl[ng][1][c32][q] +
+                               (uint32_t)svl[ng][2][c32][q] + (uint32_t)svl[ng][3][c32][q]));
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int mr = 32 * mg + 8 * (i >> 2) + 4 * half + (i & 3);
+    if (mr >= pairs) continue;
+    const int rr = mr / grp, h = g * grp + (mr - rr * grp);
+    if (h < a.h0 || h >= a.h1) continue;
+    const size_t row = (size_t)(T.r0 + rr) * a.nh + h;
+    v4i v;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      v[q] = (int)(((uint32_t)H[q][i] << 8) + (uint32_t)L[q][i] + (uint32_t)bias[q]);
+    if (a.p3_chunks == 1 && !a.dup) {
+      const float s = a.wq[row];
+      float* o = a.out + row * a.hd + d0 + 4 * c32;
+#pragma unroll
+      for (int q = 0; q < 4; q++) o[q] = (float)v[q] * s;
+    } else {
+      *(v4i*)(a.part + (row * a.p3_chunks + blockIdx.z) * a.hd + d0 + 4 * c32) = v;
+    }
   }
 }
 
 // ---------------------------------------------------------------- 4. final
-// grid (m * (h1 - h0), hd / 64), 64 threads: one dim per thread, all of the
-// row's chunk partials in flight at once (at most 32); out = (float)(their
-// sum) * (wmax / 65535), 0 when the weights were all zero.
-__global__ __launch_bounds__(64) void attn_final_kernel(const AttnArgs a) {
+// grid (m * (h1 - h0)), hd / 4 threads (a multiple of 16), four dims each: the
+// chunks' partial sums, plus once more the slots that the row counts twice.
+__global__ __launch_bounds__(128) void attn_final_kernel(const AttnArgs a) {
   const int nhr = a.h1 - a.h0;
   const int r = blockIdx.x / nhr, h = a.h0 + ((int)blockIdx.x - r * nhr);
-  const int grp = a.nh / a.kvh, g = h / grp, hl = h - g * grp;
-  const Geo G = row_geo(a, r);
-  const int nchunk = max(1, (G.dom_steps + 4 * a.p3_spw - 1) / (4 * a.p3_spw));
-  const int i = 64 * blockIdx.y + threadIdx.x;
-  const int32_t* part = a.part + (size_t)(r * a.kvh + g) * a.p3_chunks * grp * a.hd + (size_t)hl * a.hd + i;
-  const size_t cs = (size_t)grp * a.hd;
-  uint32_t v[32];
+  const int d = 4 * threadIdx.x;
+  const size_t row = (size_t)r * a.nh + h;
+  const int32_t* part = a.part + row * a.p3_chunks * a.hd + d;
+  uint32_t t[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int c = 0; c < a.p3_chunks; c++) {
+    const v4i v = *(const v4i*)(part + (size_t)c * a.hd);
 #pragma unroll
-  for (int c = 0; c < 32; c++) v[c] = c < nchunk ? (uint32_t)part[c * cs] : 0u;
-  uint32_t t = 0;  // integer sum: any order gives the same bits
+    for (int q = 0; q < 4; q++) t[q] += (uint32_t)v[q];
+  }
+  if (a.dup) {
+    const int grp = a.nh / a.kvh, g = h / grp, hl = h - g * grp;
+    const int si = seq_of(a, a.row0, r);
+    const KernArgs ka = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    const int dr = r - ka->seq[si].row0;
+    const Geo G = seq_geo(a, si, dr, 1);
+    const int t0 = dr / a.rt * a.rt;
+    const Geo T = seq_geo(a, si, t0, min(a.rt, ka->seq[si].nrows - t0));
+    int plane;
+    const int8_t* wp = planes(a, T, r, g, hl, &plane);
+    const int kvd = a.kvh * a.hd;
+    for (int s = G.lo0; s < min(G.hi1, G.ring); s++) {
+      const int o = T.dom_off(s);
+      const int8_t* p = wp + (size_t)(o >> 5) * (2 * plane) + (o & 31);
+      const uint32_t iw = 256u * (uint8_t)(p[0] ^ 0x80) + (uint8_t)(p[plane] ^ 0x80);
+      const int8_t* v = G.vc + ((size_t)(s >> 2) * kvd + g * a.hd + d) * 4 + (s & 3);
 #pragma unroll
-  for (int c = 0; c < 32; c++) t += v[c];
-  a.out[((size_t)r * a.nh + h) * a.hd + i] = (float)(int32_t)t * a.wq[r * a.nh + h];
+      for (int q = 0; q < 4; q++) t[q] += iw * (uint32_t)(int32_t)v[4 * q];
+    }
+  }
+  float* o = a.out + row * a.hd + d;
+  const float s = a.wq[row];
+#pragma unroll
+  for (int q = 0; q < 4; q++) o[q] = (float)(int32_t)t[q] * s;
 }
 
 // ------------------------------------------------------ single-launch path
@@ -519,7 +888,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fused_kernel(const AttnArgs a) {
   float* smax = wqs + 16;   // [head][wave]: the maximum score
   float* wred = smax + 128; // per wave: the maximum weight of its head
   float* E = wred + 16;
-  int8_t* PL = (int8_t*)E + fused_e_bytes(NW, hpw, a.max_n);
+  int8_t* PL = (int8_t*)E + fused_e_bytes(NW, hpw, a.max_n);  // three 7-bit planes, iw = a 2^14 + b 2^7 + c
   const int kvd = a.kvh * HD;
   const int c16 = lane & 15, q4 = lane >> 4;
 
@@ -797,49 +1166,82 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const float* k, const flo
   if (tid == 0) (isv ? vs : ks)[slot] = sc;
 }
 
-template <int KS>
-hipError_t launch_scores(const AttnArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL(attn_scores_kernel<KS>, dim3(a.p1_chunks, a.m * a.kvh), dim3(256), 0, st, a);
+// f(integral_constant<head_dim / 64>)
+template <class F>
+hipError_t with_ks(int hd, F&& f) {
+  switch (hd / 64) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    case 4: return f(std::integral_constant<int, 4>{});
+    case 5: return f(std::integral_constant<int, 5>{});
+    case 6: return f(std::integral_constant<int, 6>{});
+    case 7: return f(std::integral_constant<int, 7>{});
+    case 8: return f(std::integral_constant<int, 8>{});
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int NQ>
+hipError_t launch_softmax(const AttnArgs& a, int T, size_t lds, hipStream_t st) {
+  static hipError_t attr = hipFuncSetAttribute((const void*)attn_softmax_kernel<NQ>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(attn_softmax_kernel<NQ>, dim3(a.m * (a.h1 - a.h0)), dim3(T), lds, st, a);
   return hipGetLastError();
+}
+
+// groups of four slots per thread: the smallest instance that covers them
+hipError_t launch_softmax(const AttnArgs& a, hipStream_t st) {
+  const int quads = 16 * a.tile_steps;
+  // with hundreds of (row, head) pairs several workgroups share a CU; a few
+  // get the widest workgroups
+  const int T = a.m * (a.h1 - a.h0) >= 256 && quads <= 6 * 512 ? 512 : 1024;
+  const int S = (((a.max_n + 15) >> 4) + 16 + 63) / 64 * 64 + 4;
+  const size_t lds = ((size_t)16 * S + 32) * 4;
+  const int nq = (quads + T - 1) / T;
+  if (nq <= 1) return launch_softmax<1>(a, T, lds, st);
+  if (nq <= 2) return launch_softmax<2>(a, T, lds, st);
+  if (nq <= 3) return launch_softmax<3>(a, T, lds, st);
+  if (nq <= 4) return launch_softmax<4>(a, T, lds, st);
+  if (nq <= 6) return launch_softmax<6>(a, T, lds, st);
+  if (nq <= 9) return launch_softmax<9>(a, T, lds, st);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
 
 size_t fgm_attn_layout(AttnArgs* a, void* base, int m, int nh, int kvh, int hd, int max_span) {
   const int grp = nh / kvh;
-  const int sc_stride = (max_span + 63) / 64 * 64;
-  // a domain spans at most max_span + 3 slots from a 64-aligned start
-  const int wpl_blocks = ((max_span + 3 + 63) / 64 + 1) * 4;
-  const int chunks = attn_pv_chunks(m, kvh, hd);
+  // the domain of a row tile: the union of its rows' ranges, at most
+  // max_span + FGM_ATTN_TILE - 1 positions, in two runs of partial steps
+  const int cap = (max_span + FGM_ATTN_TILE + 6) / 64 + 4;
   auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
   size_t off = 0;
   const size_t o_sc = off;
-  off = al(off + (size_t)m * nh * sc_stride * 4);
+  off = al(off + (size_t)m * nh * cap * 64 * 4);
   const size_t o_wpl = off;
-  off = al(off + (size_t)m * kvh * wpl_blocks * 48 * grp);
+  off = al(off + (size_t)m * kvh * grp * cap * 128);
   const size_t o_part = off;
-  off = al(off + (size_t)m * kvh * chunks * grp * hd * 4);
+  off = al(off + (size_t)attn_part_rows(m) * nh * hd * 4);
   const size_t o_wq = off;
   off = al(off + (size_t)m * nh * 4);
   if (a && base) {
     char* b = (char*)base;
     a->sc = (float*)(b + o_sc);
-    a->sc_stride = sc_stride;
+    a->cap = cap;
     a->wpl = (int8_t*)(b + o_wpl);
-    a->wpl_blocks = wpl_blocks;
     a->part = (int32_t*)(b + o_part);
-    a->p3_chunks = chunks;
     a->wq = (float*)(b + o_wq);
   }
   return off;
 }
 
 hipError_t fgm_launch_attn(const AttnArgs& a, hipStream_t st) {
-  const int max_n = a.max_n;
   if (a.m <= 0 || a.h1 <= a.h0) return hipSuccess;
   hipError_t e = hipSuccess;
   // one launch when every row is short and a kv group fits the workgroup;
-  // FGM_ATTN_FUSED=0 keeps the four-launch path (for comparison and tests)
+  // FGM_ATTN_FUSED=0 keeps the longer path (for comparison and tests)
   const int grp = a.nh / a.kvh;
   const char* fz = getenv("FGM_ATTN_FUSED");
   // query heads per workgroup: as few as fill the chip (256 CUs) once
@@ -848,48 +1250,47 @@ hipError_t fgm_launch_attn(const AttnArgs& a, hipStream_t st) {
   while (f.hpw < grp && a.m * a.kvh * ((grp + f.hpw - 1) / f.hpw) > 256) f.hpw *= 2;
   f.hpw = std::min(f.hpw, grp);
   const size_t flds = fused_lds(fused_waves(a.hd), a.hd, f.hpw, a.max_n, a.max_steps);
-  if (a.max_n <= FUSED_MAX_N && grp <= FUSED_MAX_GRP && !(fz && fz[0] == '0') && flds <= 160 * 1024) {
-    switch (a.hd / 64) {
-      case 1: return launch_fused<1>(f, flds, st);
-      case 2: return launch_fused<2>(f, flds, st);
-      case 3: return launch_fused<3>(f, flds, st);
-      case 4: return launch_fused<4>(f, flds, st);
-      case 5: return launch_fused<5>(f, flds, st);
-      case 6: return launch_fused<6>(f, flds, st);
-      case 7: return launch_fused<7>(f, flds, st);
-      case 8: return launch_fused<8>(f, flds, st);
-      default: return hipErrorInvalidValue;
-    }
+  if (a.max_n <= FUSED_MAX_N && grp <= FUSED_MAX_GRP && !(fz && fz[0] == '0') && flds <= 160 * 1024)
+    return with_ks(a.hd, [&](auto ks) { return launch_fused<decltype(ks)::value>(f, flds, st); });
+
+  const int chunks = (a.tile_steps + a.p1_steps - 1) / a.p1_steps;
+  if (a.rt > 1) {
+    const int pairs = a.m * a.nh;
+    hipLaunchKernelGGL(attn_quant_q_kernel, dim3((pairs + 3) / 4), dim3(256), 0, st, a.q, (int8_t*)a.part, a.wq, pairs,
+                       a.hd);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    e = with_ks(a.hd, [&](auto ks) {
+      hipLaunchKernelGGL(attn_scores_tile_kernel<decltype(ks)::value>, dim3(chunks, a.ntiles * a.kvh), dim3(256), 0, st,
+                         a);
+      return hipGetLastError();
+    });
+  } else {
+    e = with_ks(a.hd, [&](auto ks) {
+      hipLaunchKernelGGL(attn_scores_kernel<decltype(ks)::value>, dim3(chunks, a.m * a.kvh), dim3(256), 0, st, a);
+      return hipGetLastError();
+    });
   }
-  if (max_n > 0) {
-    switch (a.hd / 64) {
-      case 1: e = launch_scores<1>(a, st); break;
-      case 2: e = launch_scores<2>(a, st); break;
-      case 3: e = launch_scores<3>(a, st); break;
-      case 4: e = launch_scores<4>(a, st); break;
-      case 5: e = launch_scores<5>(a, st); break;
-      case 6: e = launch_scores<6>(a, st); break;
-      case 7: e = launch_scores<7>(a, st); break;
-      case 8: e = launch_scores<8>(a, st); break;
-      default: return hipErrorInvalidValue;
-    }
-    if (e != hipSuccess) return e;
+  if (e != hipSuccess) return e;
+  if ((e = launch_softmax(a, st)) != hipSuccess) return e;
+  if (a.rt > 1) {
+    const dim3 grid((a.hd + 255) / 256, a.ntiles * a.kvh, a.p3_chunks);
+    if (a.hd > 128)
+      hipLaunchKernelGGL(attn_pv_tile_kernel<2>, grid, dim3(512), 0, st, a);
+    else
+      hipLaunchKernelGGL(attn_pv_tile_kernel<1>, grid, dim3(256), 0, st, a);
+  } else {
+    const dim3 grid(a.hd / 32, a.m * a.kvh, a.p3_chunks);
+    if (grp > 8)
+      hipLaunchKernelGGL(attn_pv_kernel<true>, grid, dim3(512), 0, st, a);
+    else
+      hipLaunchKernelGGL(attn_pv_kernel<false>, grid, dim3(1024), 0, st, a);
   }
-  static hipError_t attr = hipFuncSetAttribute((const void*)attn_softmax_kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  if (attr != hipSuccess) return attr;
-  // long rows with few (row, head) pairs get the widest workgroups; with
-  // hundreds of pairs the chip is full anyway
-  const int nwg = a.m * (a.h1 - a.h0);
-  const int T = max_n <= 1024 ? 256 : (max_n >= 4096 && nwg < 256 ? 1024 : 512);
-  const int S = (((max_n + 15) >> 4) + 16 + 63) / 64 * 64 + 4;
-  const size_t lds = ((size_t)16 * S + 32) * 4;
-  hipLaunchKernelGGL(attn_softmax_kernel, dim3(a.m * (a.h1 - a.h0)), dim3(T), lds, st, a);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(attn_pv_kernel, dim3(a.p3_chunks, a.hd / 64, a.m * a.kvh), dim3(256), 0, st, a);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(attn_final_kernel, dim3(a.m * (a.h1 - a.h0), a.hd / 64), dim3(64), 0, st, a);
-  return hipGetLastError();
+  if (a.p3_chunks > 1 || a.dup) {
+    hipLaunchKernelGGL(attn_final_kernel, dim3(a.m * (a.h1 - a.h0)), dim3(a.hd / 4), 0, st, a);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 hipError_t fgm_launch_store_v_t(int8_t* vt, const int8_t* src, int n, int slot, hipStream_t st) {

@@ -129,24 +129,28 @@ struct AttnSeq {
 };
 struct AttnArgs {
   AttnSeq seq[FGM_ATTN_MAX_SEQ];
-  int row0[FGM_ATTN_MAX_SEQ];  // seq[i].row0, INT_MAX past nseq (ascending: row r is in the last i with row0[i] <= r)
+  int row0[FGM_ATTN_MAX_SEQ];   // seq[i].row0, INT_MAX past nseq (ascending: row r is in the last i with row0[i] <= r)
+  int tile0[FGM_ATTN_MAX_SEQ];  // the sequence's first row tile, INT_MAX past nseq
   int nseq, m, nh, kvh, hd, window, h0, h1;
   int one_row;           // every sequence has exactly one row
   int max_n, max_steps;  // over the rows: positions, P.V slot steps
   int hpw;               // query heads per workgroup (single-launch path)
+  // Rows of one sequence share their reads of K and V in tiles of rt
+  // consecutive rows (rt = 1: every row by itself).  A tile's rows share one
+  // slot domain, that of the union of their ranges.
+  int rt, ntiles, tile_steps;  // tile_steps: the largest domain, in 64-slot steps
+  int dup;                     // some row counts a slot group twice (AttnSpan)
   float* out;
   const float* q;
   // scratch
-  float* sc;          // scores / exponentials [m][nh][sc_stride]
-  int sc_stride;
-  int8_t* wpl;        // weight planes [m][kvh][wpl_blocks][3][grp][16]
-  int wpl_blocks;
-  int32_t* part;      // P.V partial sums [m][kvh][p3_chunks][grp][hd]
-  float* wq;          // per (row, head) dequantisation step, 0 = zero output
-  int p1_chunk;       // positions per score workgroup
-  int p1_chunks;      // score workgroups per (row, kv head) in the grid
-  int p3_spw;         // 64-slot steps per wave in a P.V workgroup
-  int p3_chunks;      // P.V slot chunks (4 * p3_spw steps) per (row, kv head)
+  float* sc;          // scores [m][nh][64 cap], by domain offset
+  int cap;            // 64-slot steps that a row's scratch holds
+  int8_t* wpl;        // weights, 128 bytes per (row, head) and step, tile by tile ([kvh][m] rows)
+  int32_t* part;      // P.V partial sums [m][nh][p3_chunks][hd]; before them, int8 queries [m][nh][hd]
+  float* wq;          // per (row, head): query scale, then the dequantisation step (0 = zero output)
+  int p1_steps;       // 64-slot steps per score workgroup
+  int p3_steps;       // 64-slot steps per P.V workgroup
+  int p3_chunks;      // P.V chunks of p3_steps
 };
 // A row's attended range and the reference's slot runs (ops.c:560-572) as
 // four-slot-aligned spans: [lo0, hi0), and [0, hi1) when the range wraps in
@@ -158,22 +162,19 @@ struct AttnArgs {
 struct AttnSpan {
   int st, en, n, s0, lo0, hi0, hi1, dom_lo, dom_steps, nst1, gap;
 };
-template <class F>  // slot_of_start(st): st % ring
-__host__ __device__ inline AttnSpan attn_span(int en, int lo, int window, int ring, F slot_of_start) {
+// The range [st, en) with st in slot s0.
+__host__ __device__ inline AttnSpan attn_span(int st, int en, int ring, int s0) {
   AttnSpan g;
-  g.en = en;
-  g.st = window > 0 ? (en - window > 0 ? en - window : 0) : lo;
-  g.n = g.en - g.st;
-  g.s0 = slot_of_start(g.st);
-  g.lo0 = g.s0 & ~3, g.hi1 = 0;
+  g.st = st, g.en = en, g.n = en - st, g.s0 = s0;
+  g.lo0 = s0 & ~3, g.hi1 = 0;
   if (ring && g.n >= ring) {  // one run over the whole ring
     g.lo0 = 0;
     g.hi0 = (ring + 3) & ~3;
-  } else if (ring && g.s0 + g.n > ring) {
+  } else if (ring && s0 + g.n > ring) {
     g.hi0 = (ring + 3) & ~3;
-    g.hi1 = (g.s0 + g.n - ring + 3) & ~3;
+    g.hi1 = (s0 + g.n - ring + 3) & ~3;
   } else {
-    g.hi0 = (g.s0 + g.n + 3) & ~3;
+    g.hi0 = (s0 + g.n + 3) & ~3;
   }
   g.nst1 = (g.hi1 + 63) >> 6, g.gap = 0;
   const int base0 = g.lo0 & ~63;
@@ -190,12 +191,14 @@ __host__ __device__ inline AttnSpan attn_span(int en, int lo, int window, int ri
   }
   return g;
 }
-// P.V slot chunks per (row, kv head): enough workgroups to fill the chip
-// (about 2048), at most 32.
-inline int attn_pv_chunks(int m, int kvh, int hd) {
-  const int per = (2048 + m * kvh * (hd / 64) - 1) / (m * kvh * (hd / 64));
-  return per < 1 ? 1 : (per > 32 ? 32 : per);
+// Start of the range of the row whose last position is en - 1.
+__host__ __device__ inline int attn_start(int en, int lo, int window) {
+  return window > 0 ? (en - window > 0 ? en - window : 0) : lo;
 }
+constexpr int FGM_ATTN_TILE = 128;  // (row, head) pairs of a row tile
+// Rows of partial sums that a scratch for m rows holds: chunks of a P.V
+// product times its rows.
+inline int attn_part_rows(int m) { return m > 1024 ? m : (32 * m < 1024 ? 32 * m : 1024); }
 // scratch layout for `m` rows whose spans (max over rows of end - start and
 // of the ring size) are at most max_span; returns the bytes and fills the
 // scratch pointers of `a` when base != nullptr.

@@ -177,6 +177,33 @@ def test_job_heads_split_and_wrapped_rings(nh, kvh, hd, cap, ring, window, pos, 
         same_or_tail_close(got[r], want, noncr)
 
 
+@pytest.mark.parametrize("nh,kvh,hd,cap,ring,window,pos,rows", [
+    (8, 1, 64, 3000, 0, 0, 2940, 60),        # row tiles of 16, the last one partial, unaligned tails
+    (3, 1, 128, 1300, 0, 0, 1100, 50),       # 42 rows a tile: 126 of its 128 pairs
+    (16, 1, 64, 1500, 1500, 1440, 4000, 9),  # 16 heads, a wrapped ring whose runs share a group
+    (8, 2, 192, 2100, 2100, 1100, 2090, 33), # a wrapped ring with a gap, three 64-dim blocks
+    (2, 2, 448, 1200, 0, 1050, 1100, 70),    # one head per kv head, window starts inside a step
+    (8, 1, 64, 32768, 0, 0, 32767, 1),       # the longest row, alone
+    (8, 1, 64, 20500, 0, 0, 20490, 5),       # long rows in a tile
+    (16, 1, 128, 1400, 1400, 1397, 2799, 3), # single rows of 16 heads, both runs in one group
+])
+def test_job_row_tiles_and_long_rows(nh, kvh, hd, cap, ring, window, pos, rows):
+    """Rows past the single-launch path: row tiles sharing K and V, single rows,
+    the walk over their slot domain."""
+    t = H.torch()
+    print(f"attn long rows {rows} heads {nh} hd {hd} ring {ring}", flush=True)
+    q, kv = cases.attn_inputs(f"long{rows}", nh, kvh, hd, cap, 1.0)
+    qrows = np.stack([np.roll(q, 17 * r) for r in range(rows)])
+    out = t.full((rows * nh * hd,), 7.0, dtype=t.float32, device="cuda")
+    K.attend(out, H.dev(qrows.reshape(-1)), [(*dev_kv(kv), cap, ring, pos, rows)], nh, kvh, hd, window)
+    got = H.host(out).reshape(rows, nh * hd)
+    for r in range(rows):
+        en = pos + r + 1
+        st = max(en - window, 0) if window else 0
+        want, noncr = oracle_out("heads", qrows[r], kv, nh, st, en, 0, nh, ring, 0.0)
+        same_or_tail_close(got[r], want, noncr)
+
+
 def test_kv_store_matches_reference_write_path():
     """fgm_hip_kv_store_dev equals quant_act + store_v_t per row (the forward
     pass's write, forward.rs:515-548), linear and wrapping ring."""
