@@ -284,19 +284,16 @@ __global__ __launch_bounds__(64 * WGM * WGN * KW) void gemm_kernel(GemmBatch bt)
 
   // The multiplies of one k-block (register set cur) with the next k-block's
   // fragment reads and one DMA part of a refill placed between them, so that
-  // LDS latency and load issue hide behind the matrix cores.  An int4 group
-  // starts from a zero accumulator (every k-block when the group is 64).
-  auto mma = [&](auto setc, bool fresh, int rs, int rslot, int rj, const char* nst) {
+  // LDS latency and load issue hide behind the matrix cores.  A 64-wide int4
+  // group starts from a zero accumulator every k-block, a wider one where the
+  // drain left it.
+  auto mma = [&](auto setc, int rs, int rslot, int rj, const char* nst) {
     constexpr int cur = decltype(setc)::value;
     sfor<0, NM>([&](auto mc) {
       constexpr int m = decltype(mc)::value;
       constexpr int s = m / (WMT * WNT), x = (m / WNT) % WMT, y = m % WNT;
-      if constexpr (BITS == 4 && s == 0) {
-        if constexpr (G1) acc[x][y] = mfma32(af[cur][0][x], bf[cur][0][y], v16i{});
-        else acc[x][y] = mfma32(af[cur][0][x], bf[cur][0][y], fresh ? v16i{} : acc[x][y]);
-      } else {
-        acc[x][y] = mfma32(af[cur][s][x], bf[cur][s][y], acc[x][y]);
-      }
+      if constexpr (G1 && s == 0) acc[x][y] = mfma32(af[cur][0][x], bf[cur][0][y], v16i{});
+      else acc[x][y] = mfma32(af[cur][s][x], bf[cur][s][y], acc[x][y]);
       if constexpr (m == 0) issue_part(rs, rslot, rj);
       sfor<m * NG / NM, (m + 1) * NG / NM>(
           [&](auto gc) { fetch_grp(std::integral_constant<int, cur ^ 1>{}, gc, nst); });
@@ -304,7 +301,10 @@ __global__ __launch_bounds__(64 * WGM * WGN * KW) void gemm_kernel(GemmBatch bt)
     });
   };
   // int4: at the end of a scale group, fold the group's sums into the fp32
-  // chain (or dump them raw)
+  // chain (or dump them raw); wider groups then start from zero (here, once a
+  // group: choosing the multiply's addend by k-block took as many VALU
+  // instructions per k-block as half a fold: N = 8192, K = 2048, group 128
+  // at M = 64 / 256 / 512 12.8 / 17.8 / 20.8 -> 11.5 / 16.4 / 18.6 us)
   auto drain = [&](auto setc, int kb) {
     constexpr int cur = decltype(setc)::value;
     if (BITS != 4 || kb >= KB || ((kb + 1) % gk) != 0) return;
@@ -327,6 +327,12 @@ __global__ __launch_bounds__(64 * WGM * WGN * KW) void gemm_kernel(GemmBatch bt)
 #pragma unroll
           for (int r = 0; r < 16; r++) cf[x][y][r] = __builtin_fmaf((float)acc[x][y][r], sc, cf[x][y][r]);
       }
+    }
+    if constexpr (!G1) {
+#pragma unroll
+      for (int x = 0; x < WMT; x++)
+#pragma unroll
+        for (int y = 0; y < WNT; y++) acc[x][y] = v16i{};
     }
   };
 
@@ -365,14 +371,13 @@ __global__ __launch_bounds__(64 * WGM * WGN * KW) void gemm_kernel(GemmBatch bt)
       const int sidx = sb + u;
       if (sidx < NSTG) {
         const int kb = (sidx * KW + kg) * KS + j;
-        const bool fresh = BITS == 4 && (kb % gk) == 0;
         if constexpr (j + 1 < KS) {
-          mma(std::integral_constant<int, cur>{}, fresh, sidx - 1 + NS, prev, j + 1,
+          mma(std::integral_constant<int, cur>{}, sidx - 1 + NS, prev, j + 1,
               gring + slot * C::STAGE + (j + 1) * C::KBLK);
         } else {
           wait_vm<(NS - 2) * C::U>();
           __syncthreads();
-          mma(std::integral_constant<int, cur>{}, fresh, sidx + NS, slot, 0, gring + next * C::STAGE);
+          mma(std::integral_constant<int, cur>{}, sidx + NS, slot, 0, gring + next * C::STAGE);
         }
         drain(std::integral_constant<int, cur>{}, kb);
       }

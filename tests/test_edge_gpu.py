@@ -74,6 +74,30 @@ def test_empty_contraction_writes_zeros_in_range_only(kind, M):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("M,N,Kd,group,n0,n1", [
+    (2033, 4096, 192, 64, 0, 256),     # 16 x 32 tiles of 128 x 128: ragged rows, an odd number of k-blocks
+    (2048, 4224, 384, 128, 4, 260),    # two k-blocks a group, columns inside the weight
+    (2048, 4096, 512, 256, 0, 256),
+    (513, 2048, 320, 320, 0, 128),     # 128 x 64 tiles, one group over all of K
+    (70, 512, 448, 64, 0, 32),         # 64 x 32 tiles
+    (70, 512, 768, 384, 0, 32),
+])
+def test_dense_int4_tiles_and_groups(M, N, Kd, group, n0, n1):
+    """The int4 tiles' row and column ends and the folds of 64-wide and wider
+    scale groups, on the rows at the ends of the m-tiles."""
+    print("q4g", M, N, Kd, group, flush=True)
+    A = oracle.gen_i8(27 + Kd, M * Kd, -127, 127).reshape(M, Kd)
+    a_s = oracle.gen_uniform(28 + Kd, M, 1e-3, 1e-2)
+    B = oracle.gen_u8(29 + Kd, N * Kd // 2)
+    bs = oracle.gen_uniform(30 + Kd, (Kd // group) * N, 5e-3, 5e-2).astype(np.float16).view(np.uint16)
+    got = H.gpu_gemm("q4g", M, N, Kd, oracle.pack_a(M, Kd, A), a_s, B, bs, group, n0, n1, fill=7.0)
+    rows = sorted({r for r in (0, 31, 32, 63, 64, 127, 128, 512, M // 2, M - 1) if r < M})
+    want = np.full((len(rows), N), 7.0, np.float32)
+    oracle.gemm_q4g(len(rows), N, Kd, oracle.pack_a(len(rows), Kd, A[rows].copy()), a_s[rows].copy(), B, bs, group,
+                    want, N, n0, n1)
+    assert _bits_equal(got[rows], want)
+
+
 @pytest.mark.parametrize("M,N,Kd", [(2048, 2048, 4160), (256, 2048, 576), (256, 2048, 1088), (256, 512, 8256)])
 def test_dense_odd_k_blocks(M, N, Kd):
     """K = 64 * odd: the K-group variants end on stages of zero-padded
