@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import enum
 import os
+import sys
 
 import numpy as np
 
@@ -52,15 +53,47 @@ def backend() -> Backend:
 
 
 # ------------------------------------------------------------------ helpers
+# A decode step is some twenty-five of these calls a layer, each a few
+# microseconds of GPU work, so what a call costs the host counts: the plain
+# cases (numpy arrays, torch.Tensor itself) are told apart by type identity,
+# and the raw stream handle is read without building a Stream object (a linear
+# of two calls 15.9 -> 10.6 us a pass, a decode step of 104 calls
+# 743 -> 507 us).
+class _Torch:
+    """What the device path needs of torch, looked up on first use."""
+
+    Tensor = current_device = raw_stream = None
+
+
+def _torch() -> None:
+    import torch
+    _Torch.current_device = staticmethod(torch.cuda.current_device)
+    _Torch.raw_stream = staticmethod(getattr(torch._C, "_cuda_getCurrentRawStream", None) or
+                                     (lambda dev: torch.cuda.current_stream(dev).cuda_stream))
+    _Torch.Tensor = torch.Tensor
+
+
 def _is_dev(x) -> bool:
-    return type(x).__module__.startswith("torch") and x.is_cuda
+    t = type(x)
+    if t is np.ndarray:
+        return False
+    if t is _Torch.Tensor:
+        return x.is_cuda
+    return t.__module__.startswith("torch") and x.is_cuda
 
 
 def _kind(*bufs) -> str:
-    kinds = {("dev" if _is_dev(b) else "host") for b in bufs if b is not None}
-    if len(kinds) != 1:
+    dev = host = False
+    for b in bufs:
+        if b is None:
+            continue
+        if _is_dev(b):
+            dev = True
+        else:
+            host = True
+    if dev == host:
         raise TypeError("pass either all numpy arrays or all GPU torch tensors")
-    return kinds.pop()
+    return "dev" if dev else "host"
 
 
 def _hp(a: np.ndarray) -> int:
@@ -76,8 +109,10 @@ def _dp(t) -> int:
 
 
 def _stream():
-    import torch
-    return torch.cuda.current_stream().cuda_stream
+    """torch's current stream on the current device, as a raw handle."""
+    if _Torch.Tensor is None:
+        _torch()
+    return _Torch.raw_stream(_Torch.current_device())
 
 
 def _len(x) -> int:
@@ -204,6 +239,12 @@ def acc_q4g(m, n, k, a, bq, group, acc, ldacc, n0, n1) -> None:
                                     _stream()))
 
 
+def _package():
+    """The package itself, whose structures are defined after this module is
+    imported."""
+    return sys.modules[__package__]
+
+
 def _ptr_or_none(t):
     return None if t is None else _dp(t)
 
@@ -213,29 +254,29 @@ def gemm_batch(problems, stream=None) -> None:
 
     `problems`: iterable of dicts with keys bits (4 or 8), m, n, k, a, a_scale,
     b, b_scale, c, ldc, n0, n1 and, for bits == 4, group."""
-    from . import GemmDesc
+    desc = _package().GemmDesc
     probs = list(problems)
-    arr = (GemmDesc * max(1, len(probs)))()
-    for i, p in enumerate(probs):
-        assert p["k"] % 64 == 0 and p["n"] % 16 == 0
-        assert (p["n1"] - p["n0"]) % 4 == 0, "n-block range must be a multiple of 4"
-        arr[i] = GemmDesc(p["bits"], p["m"], p["n"], p["k"], p.get("group", 64), _dp(p["a"]),
-                          _dp(p["a_scale"]), _dp(p["b"]), _dp(p["b_scale"]), _dp(p["c"]),
-                          p["ldc"], p["n0"], p["n1"])
+    arr = (desc * max(1, len(probs)))()
+    for d, p in zip(arr, probs):
+        n, k, n0, n1 = p["n"], p["k"], p["n0"], p["n1"]
+        assert k % 64 == 0 and n % 16 == 0
+        assert (n1 - n0) % 4 == 0, "n-block range must be a multiple of 4"
+        d.__init__(p["bits"], p["m"], n, k, p.get("group", 64), _dp(p["a"]), _dp(p["a_scale"]), _dp(p["b"]),
+                   _dp(p["b_scale"]), _dp(p["c"]), p["ldc"], n0, n1)
     check(lib().fgm_hip_gemm_batch_dev(arr, len(probs), _stream() if stream is None else stream))
 
 
 def prep_batch(problems, stream=None) -> None:
     """fgm_prep_rows for several device activations in one launch.  Each dict:
     src, lda, rot, qa, qs, pa, m, k, hsz, r0, r1 (rot / qa may be None)."""
-    from . import PrepDesc
+    desc = _package().PrepDesc
     probs = list(problems)
-    arr = (PrepDesc * max(1, len(probs)))()
-    for i, p in enumerate(probs):
+    arr = (desc * max(1, len(probs)))()
+    for d, p in zip(arr, probs):
         assert p["r0"] % 16 == 0, "prep row start must be tile-aligned"
-        arr[i] = PrepDesc(_dp(p["src"]), p["lda"], _ptr_or_none(p.get("rot")),
-                          _ptr_or_none(p.get("qa")), _dp(p["qs"]), _dp(p["pa"]), p["m"], p["k"],
-                          p.get("hsz", 0), p["r0"], p["r1"])
+        d.__init__(_dp(p["src"]), p["lda"], _ptr_or_none(p.get("rot")),
+                   _ptr_or_none(p.get("qa")), _dp(p["qs"]), _dp(p["pa"]), p["m"], p["k"],
+                   p.get("hsz", 0), p["r0"], p["r1"])
     check(lib().fgm_hip_prep_batch_dev(arr, len(probs), _stream() if stream is None else stream))
 
 
