@@ -64,6 +64,14 @@ FGM_DEV float wave_max(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// max of three without the quieting of signalling NaNs (results of arithmetic
+// are never signalling)
+FGM_DEV float max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
 // max over the workgroup; `red` holds one float per wave; every thread gets it
 FGM_DEV float block_max(float v, float* red) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -435,12 +443,15 @@ __global__ __launch_bounds__(256, 2) void attn_scores_tile_kernel(const AttnArgs
 // the ordered sum: e[16 c + j] at lds[j * S + c] (S = 4 mod 64, >= n / 16 +
 // 16), then the reduction slots.  A few rows are one dependent chain (8 rows x
 // 8 heads x 8192 positions: 15.2 us walking LDS, 9.5 us from registers); many
-// are bound by VALU issue, about 60 instructions a slot (2048 pairs x 8192:
-// 72 -> 42 us).
+// wait for their own barriers, loads and ordered sum about half the time
+// (2048 pairs x 8192: 72 us walking LDS, 42 us from registers with three
+// workgroups per CU and 54 VALU instructions a slot; 35 us with four, the V
+// scales loaded after the exponentials to fit their registers, and fewer
+// instructions).
 FGM_DEV int exp_stride(int n) { return (((n + 15) >> 4) + 16 + 63) / 64 * 64 + 4; }
 
-template <int NQ>
-__global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
+template <int NQ, int T_>  // T_ = 512, NQ <= 4: four workgroups per CU (64 registers)
+__global__ __launch_bounds__(T_, T_ == 512 && NQ <= 4 ? 8 : 4) void attn_softmax_kernel(const AttnArgs a) {
   extern __shared__ float lds[];
   const int nhr = a.h1 - a.h0;
   // consecutive (row, head) pairs on one XCD: they share lines of the weights
@@ -465,25 +476,27 @@ __global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
   const int nq = 16 * T.dom_steps;
 
   // A wave's 64 groups j are 256 consecutive domain offsets.  Where all of
-  // them hold positions of the row before its n % 16 tail (`u0` of the first,
-  // the others in order), nothing has to be masked.  Elsewhere, slots outside
-  // the range take part in nothing: their score is -inf, their V scale and so
-  // their weight 0, and their exponential goes to a place that nobody reads.
+  // them hold positions of the row before its n % 16 tail (uc: the chunk of 16
+  // of the first; it starts at r0 % 16, the same for all j that count here),
+  // nothing has to be masked, and an LDS index is one addition.  Elsewhere,
+  // slots outside the range take part in nothing: their score is -inf, their
+  // V scale and so their weight 0, and their exponential goes to a place that
+  // nobody reads.
   const int DUMP = 16 * S + 24;
   float e[NQ][4];
-  int vs[NQ][4], u0[NQ];
+  int vs[NQ][4], uc[NQ], r0 = -1;
 #pragma unroll
   for (int j = 0; j < NQ; j++) {
     const int q0 = 64 * w + nt * j, f = T.dom_slot4(q0), l = T.dom_slot4(q0 + 63) + 3;
     const int uf = G.pos_of(f), ul = G.pos_of(l);
-    u0[j] = l - f == 255 && q0 + 64 <= nq && uf >= 0 && ul == uf + 255 && ul < n16 ? uf : -1;
+    const bool full = l - f == 255 && q0 + 64 <= nq && uf >= 0 && ul == uf + 255 && ul < n16 &&
+                      (r0 < 0 || r0 == (uf & 15));
+    if (full) r0 = uf & 15;
+    uc[j] = full ? uf >> 4 : -1;
     const int qd = tid + nt * j, s4 = T.dom_slot4(qd);
-    if (u0[j] >= 0) {
+    if (full) {
       const float4 v = *(const float4*)(scr + 4 * qd);
       e[j][0] = v.x, e[j][1] = v.y, e[j][2] = v.z, e[j][3] = v.w;
-      const v4i x = buf_load_b128(rvs, 4u * (uint32_t)s4, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++) vs[j][i] = x[i];
     } else {
       float4 v = {0, 0, 0, 0};
       if (qd < nq) v = *(const float4*)(scr + 4 * qd);
@@ -491,37 +504,45 @@ __global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const bool ok = qd < nq && (unsigned)G.pos_of(s4 + i) < (unsigned)n;
-        vs[j][i] = buf_load_b32(rvs, ok ? 4u * (uint32_t)(s4 + i) : FGM_OOB, 0);
         e[j][i] = ok ? e[j][i] : -INFINITY;
       }
     }
   }
   float mx = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < NQ; j++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) mx = __builtin_fmaxf(mx, e[j][i]);
+  for (int j = 0; j < NQ; j++) mx = max3(max3(mx, e[j][0], e[j][1]), e[j][2], e[j][3]);
   mx = block_max(mx, red);
+  // LDS indices of the groups' slots from the first full chunk on
+  int at0[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int u = r0 + 4 * lane + i;
+    at0[i] = (u & 15) * S + (u >> 4);
+  }
   uint64_t tl = 0;  // this thread's slots in the tail
 #pragma unroll
   for (int j = 0; j < NQ; j++) {
-    if (u0[j] >= 0) {
+    if (uc[j] >= 0) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int u = u0[j] + 4 * lane + i;
         e[j][i] = exp16(e[j][i] - mx);
-        lds[(u & 15) * S + (u >> 4)] = e[j][i];
+        lds[at0[i] + uc[j]] = e[j][i];
       }
+      const v4i x = buf_load_b128(rvs, 4u * (uint32_t)T.dom_slot4(tid + nt * j), 0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) vs[j][i] = x[i];
     } else {
       const int qd = tid + nt * j, s4 = T.dom_slot4(qd);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const int u = G.pos_of(s4 + i);
         const float x = e[j][i] - mx;
-        int at = qd < nq && (unsigned)u < (unsigned)n ? (u & 15) * S + (u >> 4) : DUMP;
+        const bool ok = qd < nq && (unsigned)u < (unsigned)n;
+        const int at = ok ? (u & 15) * S + (u >> 4) : DUMP;
+        vs[j][i] = buf_load_b32(rvs, ok ? 4u * (uint32_t)(s4 + i) : FGM_OOB, 0);
         e[j][i] = exp16(x);
         // the tail: shifted scores, for lanes 0..15 to exponentiate
-        const bool t = at != DUMP && u >= n16;
+        const bool t = ok && u >= n16;
         lds[at] = t ? x : e[j][i];
         tl |= (uint64_t)t << (4 * j + i);
       }
@@ -546,14 +567,15 @@ __global__ __launch_bounds__(1024) void attn_softmax_kernel(const AttnArgs a) {
         if (tl >> (4 * j + i) & 1)
           e[j][i] = lds[(G.pos_of(T.dom_slot4(tid + nt * j) + i) & 15) * S + (n16 >> 4)];
   }
-  // weights (e * inv) * vs, and their maximum
+  // weights (e * inv) * vs (the V scales in flight since the exponentials),
+  // and their maximum
   float wm = 0.0f;
 #pragma unroll
   for (int j = 0; j < NQ; j++)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       e[j][i] = (e[j][i] * inv) * __int_as_float(vs[j][i]);
-      wm = __builtin_fmaxf(wm, e[j][i]);
+      if (i & 1) wm = max3(wm, e[j][i - 1], e[j][i]);
     }
   wm = block_max(wm, red);
   const bool some = wm > 0.0f;
@@ -690,49 +712,76 @@ __global__ __launch_bounds__(TWO ? 512 : 1024) void attn_pv_kernel(const AttnArg
 // threads (NG = 2, or 1 for head_dim <= 128): the 128 pairs of a tile x 128 NG
 // dims x the chunk's steps on v_mfma_i32_32x32x32_i8.  Wave (mg, ng) takes
 // the pairs 32 mg ... and the dims 128 ng ..., with both planes' sums in
-// registers; its A operands are 16-byte loads of the planes' rows, its B
-// operands 16-byte loads [4 dims][4 slots] of V as above (column c = dim
-// 4 c + q).  The four waves of a dim block read the same V, and the NG waves
-// of a pair block the same planes, out of L1; three half steps are in flight.
+// registers.  Half steps of 32 slots go through LDS, a ring of NS filled by
+// 1 KB LDS-DMA units: the planes of 32 pairs each, and V's rows of eight slot
+// groups.  A fragments are 16 bytes of a pair's 32, B fragments the 16 bytes
+// [4 dims][4 slots] of a group, as above (column c = dim 4 c + q).  sum v: wave
+// mg adds up the half steps mg, mg + 4, ...
 // 256 rows x 8 heads x 8192 slots at head_dim 512: 93 us with every row
-// reading V for itself and three 7-bit planes, 40 us so (54 us while a pair's
-// hi and lo bytes lay side by side, 32-byte pieces of 128-byte lines).
-// sum v: wave mg adds up the half steps mg, mg + 4, ...
+// reading V for itself and three 7-bit planes; 40 us as tiles with the
+// operands loaded from L1 to registers (48 KB a half step and CU, 768 cycles
+// of L1 under 512 of the matrix cores), 37 us through LDS, both in four chunks
+// (128 workgroups); 28.5 us in eight.
 template <int NG>
 __global__ __launch_bounds__(256 * NG, 2) void attn_pv_tile_kernel(const AttnArgs a) {
+  constexpr int NW = 4 * NG, UNITS = 8 + 4 * NG, UPW = UNITS / NW, NS = 5, STAGE = UNITS * 1024;
+  static_assert(UPW * NW == UNITS, "units per wave");
+  __shared__ __attribute__((aligned(1024))) int8_t ring[NS * STAGE];
   __shared__ __attribute__((aligned(16))) int svl[NG][4][32][4];
   const int t = blockIdx.y / a.kvh, g = blockIdx.y - t * a.kvh;
   const Geo T = tile_geo(a, t);
   const int lane = threadIdx.x & 63, w = wave_id(), mg = w & 3, ng = w >> 2;
   const int grp = a.nh / a.kvh, pairs = T.nr * grp;
-  const int kvd = a.kvh * a.hd, d0 = (int)blockIdx.x * 128 * NG + 128 * ng;
+  const int kvd = a.kvh * a.hd, dwg = (int)blockIdx.x * 128 * NG, d0 = dwg + 128 * ng;
   const int c32 = lane & 31, half = lane >> 5;
+  const int first = 2 * (int)blockIdx.z * a.p3_steps, last = min(first + 2 * a.p3_steps, 2 * T.dom_steps);
   int plane;
-  const int8_t* wp = planes(a, T, T.r0, g, 0, &plane) + min(32 * mg + c32, pairs - 1) * 32 + 16 * half;
-  const __amdgpu_buffer_rsrc_t rv = make_rsrc(T.vc, (uint32_t)((size_t)((T.k_len + 3) >> 2) * kvd * 4));
+  const int8_t* wp = planes(a, T, T.r0, g, 0, &plane);
+  const v4i rw = rsrc_words(wp, (uint32_t)plane * 4u * (uint32_t)T.dom_steps);
+  const v4i rv = rsrc_words(T.vc, (uint32_t)((size_t)((T.k_len + 3) >> 2) * kvd * 4));
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)ring;
+  // DMA unit u = w + NW i of a half step: planes (u / 4) of the pairs 32 (u %
+  // 4) ... (past the tile's pairs: zeros), or V group rows, NG a unit
+  uint32_t src[UPW];
+#pragma unroll
+  for (int i = 0; i < UPW; i++) {
+    const int u = w + NW * i;
+    if (u < 8) {
+      const int o = (u & 3) * 1024 + 16 * lane;
+      src[i] = o < plane ? (uint32_t)((u >> 2) * plane + o) : FGM_OOB;
+    } else {
+      const int row = NG == 2 ? u - 8 : 2 * (u - 8) + half, o = NG == 2 ? 16 * lane : 16 * c32;
+      src[i] = ((uint32_t)row * (uint32_t)kvd + (uint32_t)(g * a.hd + dwg)) * 4u + (uint32_t)o;
+    }
+  }
+  auto issue = [&](int hs, int slot) {
+    const uint32_t gi = (uint32_t)(T.dom_slot(hs >> 1) >> 2) + 8u * (hs & 1);
+    const uint32_t av = gi * (uint32_t)kvd * 4u, aw = (uint32_t)hs * 2u * (uint32_t)plane;
+    const uint32_t to = lds0 + (uint32_t)slot * STAGE + 1024u * w;
+#pragma unroll
+    for (int i = 0; i < UPW; i++) {
+      if (w + NW * i < 8)
+        dma16(rw, to + 1024u * NW * i, src[i] == FGM_OOB ? FGM_OOB : src[i] + aw, 0);
+      else
+        dma16(rv, to + 1024u * NW * i, src[i] + av, 0);
+    }
+  };
   v16i H[4], L[4];
   int sv[4] = {0, 0, 0, 0};
 #pragma unroll
   for (int q = 0; q < 4; q++) H[q] = L[q] = v16i{};
-  const int first = 2 * (int)blockIdx.z * a.p3_steps, last = min(first + 2 * a.p3_steps, 2 * T.dom_steps);
-  // half steps of 32 slots: V groups 4 half + r of the eight, planes' bytes
-  // 32 hs + 16 half; past the last one, that one again (never multiplied)
-  auto load = [&](v4i* A, v4i* V, int hs) {
-    hs = min(hs, last - 1);
-    const uint32_t gi = (uint32_t)(T.dom_slot(hs >> 1) >> 2) + 8u * (hs & 1) + 4u * half;
-    const uint32_t at = (gi * (uint32_t)kvd + (uint32_t)(g * a.hd + d0 + 4 * c32)) * 4u;
-    const int8_t* p = wp + (size_t)hs * (2 * plane);
-    A[0] = *(const v4i*)p;
-    A[1] = *(const v4i*)(p + plane);
+  const int8_t* fa = ring + mg * 1024 + 32 * c32 + 16 * half;
+  const int8_t* fb = ring + 8192 + (NG * 512) * 4 * half + 512 * ng + 16 * c32;
+  auto mul = [&](int hs, int slot) {
+    const v4i A0 = *(const v4i*)(fa + slot * STAGE), A1 = *(const v4i*)(fa + slot * STAGE + 4096);
+    v4i V[4];
 #pragma unroll
-    for (int rr = 0; rr < 4; rr++) V[rr] = buf_load_b128(rv, at + (uint32_t)(rr * kvd * 4), 0);
-  };
-  auto mul = [&](const v4i* A, const v4i* V, int hs) {
+    for (int rr = 0; rr < 4; rr++) V[rr] = *(const v4i*)(fb + slot * STAGE + NG * 512 * rr);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const v4i b = {V[0][q], V[1][q], V[2][q], V[3][q]};
-      H[q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], b, H[q], 0, 0, 0);
-      L[q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[1], b, L[q], 0, 0, 0);
+      H[q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A0, b, H[q], 0, 0, 0);
+      L[q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1, b, L[q], 0, 0, 0);
     }
     if ((hs & 3) == mg) {
 #pragma unroll
@@ -741,20 +790,25 @@ __global__ __launch_bounds__(256 * NG, 2) void attn_pv_tile_kernel(const AttnArg
         for (int rr = 0; rr < 4; rr++) sv[q] = dot4_ones(V[rr][q], sv[q]);
     }
   };
-  if (first < last) {
-    v4i A0[2], A1[2], A2[2], V0[4], V1[4], V2[4];
-    load(A0, V0, first);
-    load(A1, V1, first + 1);
+#pragma unroll
+  for (int i = 0; i < NS - 1; i++)
+    if (first + i < last) issue(first + i, i);
+  // Half step hs is in slot (hs - first) % NS.  When its turn comes, the wave
+  // has issued at most NS - 2 later ones; the barrier then shows every wave's
+  // part, and that all are done with half step hs - 1, whose slot is refilled.
+  int hs = first;
 #pragma unroll 1
-    for (int hs = first; hs < last; hs += 3) {
-      load(A2, V2, hs + 2);
-      mul(A0, V0, hs);
-      if (hs + 1 >= last) break;
-      load(A0, V0, hs + 3);
-      mul(A1, V1, hs + 1);
-      if (hs + 2 >= last) break;
-      load(A1, V1, hs + 4);
-      mul(A2, V2, hs + 2);
+  while (hs < last) {
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      if (hs < last) {
+        if (hs + NS - 2 < last) wait_vm<(NS - 2) * UPW>();
+        else wait_vm<0>();
+        __syncthreads();
+        if (hs + NS - 1 < last) issue(hs + NS - 1, (i + NS - 1) % NS);
+        mul(hs, i);
+      }
+      hs++;
     }
   }
 #pragma unroll
@@ -1182,12 +1236,12 @@ hipError_t with_ks(int hd, F&& f) {
   }
 }
 
-template <int NQ>
-hipError_t launch_softmax(const AttnArgs& a, int T, size_t lds, hipStream_t st) {
-  static hipError_t attr = hipFuncSetAttribute((const void*)attn_softmax_kernel<NQ>,
+template <int NQ, int T>
+hipError_t launch_softmax(const AttnArgs& a, size_t lds, hipStream_t st) {
+  static hipError_t attr = hipFuncSetAttribute((const void*)attn_softmax_kernel<NQ, T>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(attn_softmax_kernel<NQ>, dim3(a.m * (a.h1 - a.h0)), dim3(T), lds, st, a);
+  hipLaunchKernelGGL((attn_softmax_kernel<NQ, T>), dim3(a.m * (a.h1 - a.h0)), dim3(T), lds, st, a);
   return hipGetLastError();
 }
 
@@ -1196,16 +1250,22 @@ hipError_t launch_softmax(const AttnArgs& a, hipStream_t st) {
   const int quads = 16 * a.tile_steps;
   // with hundreds of (row, head) pairs several workgroups share a CU; a few
   // get the widest workgroups
-  const int T = a.m * (a.h1 - a.h0) >= 256 && quads <= 6 * 512 ? 512 : 1024;
+  const bool many = a.m * (a.h1 - a.h0) >= 256 && quads <= 6 * 512;
   const int S = (((a.max_n + 15) >> 4) + 16 + 63) / 64 * 64 + 4;
   const size_t lds = ((size_t)16 * S + 32) * 4;
-  const int nq = (quads + T - 1) / T;
-  if (nq <= 1) return launch_softmax<1>(a, T, lds, st);
-  if (nq <= 2) return launch_softmax<2>(a, T, lds, st);
-  if (nq <= 3) return launch_softmax<3>(a, T, lds, st);
-  if (nq <= 4) return launch_softmax<4>(a, T, lds, st);
-  if (nq <= 6) return launch_softmax<6>(a, T, lds, st);
-  if (nq <= 9) return launch_softmax<9>(a, T, lds, st);
+  if (many) {
+    if (quads <= 1 * 512) return launch_softmax<1, 512>(a, lds, st);
+    if (quads <= 2 * 512) return launch_softmax<2, 512>(a, lds, st);
+    if (quads <= 3 * 512) return launch_softmax<3, 512>(a, lds, st);
+    if (quads <= 4 * 512) return launch_softmax<4, 512>(a, lds, st);
+    return launch_softmax<6, 512>(a, lds, st);
+  }
+  if (quads <= 1 * 1024) return launch_softmax<1, 1024>(a, lds, st);
+  if (quads <= 2 * 1024) return launch_softmax<2, 1024>(a, lds, st);
+  if (quads <= 3 * 1024) return launch_softmax<3, 1024>(a, lds, st);
+  if (quads <= 4 * 1024) return launch_softmax<4, 1024>(a, lds, st);
+  if (quads <= 6 * 1024) return launch_softmax<6, 1024>(a, lds, st);
+  if (quads <= 9 * 1024) return launch_softmax<9, 1024>(a, lds, st);
   return hipErrorInvalidValue;
 }
 

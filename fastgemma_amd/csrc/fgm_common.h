@@ -178,7 +178,7 @@ FGM_DEV void sfor(F&& f) {
 
 // exp512_ps (ops.c:21-39) on one lane: Cephes range reduction and polynomial.
 FGM_DEV float exp16(float x) {
-  x = __builtin_fminf(__builtin_fmaxf(x, -88.0f), 88.0f);
+  x = __builtin_amdgcn_fmed3f(x, -88.0f, 88.0f);  // the clamp; NaN gives -88, as max then min do
   const float fx = __builtin_rintf(x * 1.44269504088896341f);
   float z = __builtin_fmaf(-fx, 0.693359375f, x);
   z = __builtin_fmaf(-fx, -2.12194440e-4f, z);

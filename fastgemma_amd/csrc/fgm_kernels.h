@@ -197,8 +197,8 @@ __host__ __device__ inline int attn_start(int en, int lo, int window) {
 }
 constexpr int FGM_ATTN_TILE = 128;  // (row, head) pairs of a row tile
 // Rows of partial sums that a scratch for m rows holds: chunks of a P.V
-// product times its rows.
-inline int attn_part_rows(int m) { return m > 1024 ? m : (32 * m < 1024 ? 32 * m : 1024); }
+// product times its rows (eight chunks of 256 rows fill the chip).
+inline int attn_part_rows(int m) { return m > 2048 ? m : (32 * m < 2048 ? 32 * m : 2048); }
 // scratch layout for `m` rows whose spans (max over rows of end - start and
 // of the ring size) are at most max_span; returns the bytes and fills the
 // scratch pointers of `a` when base != nullptr.
