@@ -1108,9 +1108,9 @@ static int attn_plan(AttnArgs& a, int* max_span) {
   a.p1_steps = (int)std::max<long long>(1, std::min<long long>(8, (a.tile_steps * units + 511) / 512));
   // P.V: one chunk when the tiles and dims fill the chip, else as many as do
   // (and as the scratch holds)
-  const int dim_wgs = a.rt > 1 ? (a.hd + 255) / 256 : a.hd / 32;
-  const int want = a.rt > 1 ? 256 : 128;
-  int chunks = (int)((want + units * dim_wgs - 1) / (units * dim_wgs));
+  a.p3_dims = a.rt > 1 ? 256 : (units * (a.hd / 32) >= 256 ? 32 : 16);
+  const int dim_wgs = (a.hd + a.p3_dims - 1) / a.p3_dims;
+  int chunks = (int)((256 + units * dim_wgs - 1) / (units * dim_wgs));
   if (m) chunks = std::min(chunks, attn_part_rows(m) / m);
   chunks = std::max(1, std::min(chunks, a.tile_steps));
   a.p3_steps = (a.tile_steps + chunks - 1) / chunks;

@@ -604,79 +604,90 @@ constexpr uint32_t IW_BIAS = 32896u;  // 256 * 128 + 128: see the planes above
 
 FGM_DEV int dot4_ones(int x, int c) { return __builtin_amdgcn_sdot4(x, 0x01010101, c, false); }
 
-// Single rows.  grid (hd / 32, m * kvh, p3_chunks), 64 NW threads: workgroup
-// (x, y, z) takes the dims [32 x, + 32) and the steps [p3_steps z, + p3_steps)
-// of the row's domain, wave w the steps w, w + NW, ...; lane (c, q4) loads the
-// 8 bytes [2 dims][4 slots] of dims 2 c, 2 c + 1 and slot groups 4 q4 + r,
-// r = 0..3 (a 128-byte line per group): register q of the four loads is one
-// MFMA B operand (column c = dim 2 c + q).  Four steps are in flight.
-// 8 rows x 8192 slots at head_dim 512: 14.7 us and 4.9 us for the partial
-// sums' launch with 4-byte loads in 2048 workgroups; 13 us so, no partial sums.  The A operand's rows are the heads' hi planes (0..7) and lo
-// planes (8..15), with more than eight heads one operand each.  Sixteen waves
-// so that one workgroup covers all of K where 64 workgroups or more run: the
-// sums stay in the workgroup and need no further launch.
-template <bool TWO>  // more than eight heads
+// Single rows.  grid (hd / (16 DPL), m * kvh, p3_chunks), 64 NW threads:
+// workgroup (x, y, z) takes the dims [16 DPL x, + 16 DPL) and the steps
+// [p3_steps z, + p3_steps) of the row's domain, wave w the steps w, w + NW,
+// ...; lane (c, q4) loads the 4 DPL bytes [DPL dims][4 slots] of dims DPL c ..
+// and slot groups 4 q4 + r, r = 0..3: register q of the four loads is one MFMA
+// B operand (column c = dim DPL c + q).  The A operand's rows are the heads'
+// hi planes (0..7) and lo planes (8..15), with more than eight heads one
+// operand each.  PF steps are in flight, without branches around the loads
+// (past the last step they read nothing), so that the waits count them.
+// Sixteen waves so that one workgroup covers all of K where 256 or more run:
+// the sums stay in the workgroup and need no further launch.  DPL = 1 (64-byte
+// pieces of V's lines; consecutive workgroups, which share them, go to one
+// XCD) where 32-dim workgroups would leave CUs idle.  8 rows x 8192 slots at
+// head_dim 512: 14.7 us and 4.9 us for the partial sums' launch with 4-byte
+// loads in 2048 workgroups, 12.4 us as 128 workgroups of 32 dims with a branch
+// around each load, 2.2 us less so (the whole call 36.3 -> 34.0 us; 37.0 with
+// 128 workgroups and no branches, eight steps in flight as four).
+template <bool TWO, int DPL>  // TWO: more than eight heads
 __global__ __launch_bounds__(TWO ? 512 : 1024) void attn_pv_kernel(const AttnArgs a) {
-  constexpr int NW = TWO ? 8 : 16;
-  __shared__ __attribute__((aligned(16))) int32_t red[NW][17][32];
-  const int r = blockIdx.y / a.kvh, g = blockIdx.y - r * a.kvh;
+  constexpr int NW = TWO ? 8 : 16, ND = 16 * DPL, PF = 4;
+  __shared__ __attribute__((aligned(16))) int32_t red[NW][17][ND];
+  const int nx = gridDim.x, total = nx * gridDim.y;
+  int id = blockIdx.x + nx * blockIdx.y;
+  if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
+  const int rg = id / nx, r = rg / a.kvh, g = rg - r * a.kvh;
   const Geo G = row_geo(a, r);
   const int grp = a.nh / a.kvh;
   const int hb = max(a.h0, g * grp), he = min(a.h1, (g + 1) * grp);
   if (hb >= he) return;
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  const int kvd = a.kvh * a.hd, d0 = 32 * blockIdx.x;
+  const int kvd = a.kvh * a.hd, d0 = ND * (id - rg * nx);
   const int c16 = lane & 15, q4 = lane >> 4;
+  const int first = (int)blockIdx.z * a.p3_steps, last = min(first + a.p3_steps, G.dom_steps);
   int plane;
-  const int8_t* wp = planes(a, G, r, g, TWO ? c16 : c16 & 7, &plane);
-  wp += (TWO ? 0 : plane * (c16 >> 3)) + (q4 >> 1) * 2 * plane + 16 * (q4 & 1);
-  const bool live = (TWO ? c16 : c16 & 7) < grp;
+  const int8_t* wp = planes(a, G, r, g, 0, &plane);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(wp, (uint32_t)(4 * plane) * (uint32_t)G.dom_steps);
+  const int hl = TWO ? c16 : c16 & 7;
+  const uint32_t wat = (uint32_t)(32 * hl + (TWO ? 0 : plane * (c16 >> 3)) + (q4 >> 1) * 2 * plane + 16 * (q4 & 1));
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(G.vc, (uint32_t)((size_t)((G.k_len + 3) >> 2) * kvd * 4));
-  v4i D0[2], D1[2];
-  int sv[2] = {0, 0};
+  const uint32_t vat = ((uint32_t)(4 * q4) * (uint32_t)kvd + (uint32_t)(g * a.hd + d0 + DPL * c16)) * 4u;
+  v4i D0[DPL], D1[DPL];
+  int sv[DPL];
 #pragma unroll
-  for (int q = 0; q < 2; q++) D0[q] = D1[q] = v4i{0, 0, 0, 0};
-  auto load = [&](v4i* A, v2i* V, int step) {
-    const uint32_t gi = (uint32_t)(G.dom_slot(step) >> 2) + 4u * q4;
-    const uint32_t at = (gi * (uint32_t)kvd + (uint32_t)(g * a.hd + d0 + 2 * c16)) * 4u;
+  for (int q = 0; q < DPL; q++) D0[q] = D1[q] = v4i{0, 0, 0, 0}, sv[q] = 0;
+  v4i A[PF][TWO ? 2 : 1];
+  int V[PF][4][DPL];
+  auto load = [&](int i, int step) {
+    const bool ok = step < last;
+    const uint32_t wo = ok && hl < grp ? wat + (uint32_t)step * (uint32_t)(4 * plane) : FGM_OOB;
+    const uint32_t vo = ok ? vat + (uint32_t)(G.dom_slot(step) >> 2) * (uint32_t)(kvd * 4) : FGM_OOB;
+    A[i][0] = buf_load_b128(rw, wo, 0);
+    if constexpr (TWO) A[i][1] = buf_load_b128(rw, wo + (uint32_t)plane, 0);
 #pragma unroll
-    for (int rr = 0; rr < 4; rr++) V[rr] = buf_load_b64(rv, at + (uint32_t)(rr * kvd * 4), 0);
-    A[0] = A[1] = v4i{0, 0, 0, 0};
-    if (live) {
-      A[0] = *(const v4i*)(wp + (size_t)step * (4 * plane));
-      if constexpr (TWO) A[1] = *(const v4i*)(wp + (size_t)step * (4 * plane) + plane);
+    for (int rr = 0; rr < 4; rr++) {
+      if constexpr (DPL == 1) {
+        V[i][rr][0] = buf_load_b32(rv, vo + (uint32_t)(rr * kvd * 4), 0);
+      } else {
+        const v2i x = buf_load_b64(rv, vo + (uint32_t)(rr * kvd * 4), 0);
+        V[i][rr][0] = x[0], V[i][rr][DPL - 1] = x[1];
+      }
     }
   };
-  auto mul = [&](const v4i* A, const v2i* V) {
+  auto mul = [&](int i) {
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const v4i b = {V[0][q], V[1][q], V[2][q], V[3][q]};
-      D0[q] = mfma16(A[0], b, D0[q]);
-      if constexpr (TWO) D1[q] = mfma16(A[1], b, D1[q]);
+    for (int q = 0; q < DPL; q++) {
+      const v4i b = {V[i][0][q], V[i][1][q], V[i][2][q], V[i][3][q]};
+      D0[q] = mfma16(A[i][0], b, D0[q]);
+      if constexpr (TWO) D1[q] = mfma16(A[i][TWO ? 1 : 0], b, D1[q]);
 #pragma unroll
       for (int rr = 0; rr < 4; rr++) sv[q] = dot4_ones(b[rr], sv[q]);
     }
   };
-  const int first = (int)blockIdx.z * a.p3_steps, last = min(first + a.p3_steps, G.dom_steps);
-  v4i A[4][2];
-  v2i V[4][4];
-  int step = first + w;
 #pragma unroll
-  for (int i = 0; i < 4; i++)
-    if (step + NW * i < last) load(A[i], V[i], step + NW * i);
+  for (int i = 0; i < PF; i++) load(i, first + w + NW * i);
 #pragma unroll 1
-  while (step < last) {
+  for (int step = first + w; step < last; step += PF * NW) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      if (step < last) {
-        mul(A[i], V[i]);
-        if (step + 4 * NW < last) load(A[i], V[i], step + 4 * NW);
-      }
-      step += NW;
+    for (int i = 0; i < PF; i++) {
+      mul(i);
+      load(i, step + (PF + i) * NW);
     }
   }
 #pragma unroll
-  for (int q = 0; q < 2; q++) {
+  for (int q = 0; q < DPL; q++) {
     sv[q] += __shfl_xor(sv[q], 16, 64);
     sv[q] += __shfl_xor(sv[q], 32, 64);
   }
@@ -684,17 +695,17 @@ __global__ __launch_bounds__(TWO ? 512 : 1024) void attn_pv_kernel(const AttnArg
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int row = 4 * q4 + i;
-    v2i v;
 #pragma unroll
-    for (int q = 0; q < 2; q++)
-      v[q] = TWO ? (int)(((uint32_t)D0[q][i] << 8) + (uint32_t)D1[q][i])
-                 : (int)(row < 8 ? (uint32_t)D0[q][i] << 8 : (uint32_t)D0[q][i]);
-    *(v2i*)&red[w][row][2 * c16] = v;
+    for (int q = 0; q < DPL; q++)
+      red[w][row][DPL * c16 + q] = TWO ? (int)(((uint32_t)D0[q][i] << 8) + (uint32_t)D1[q][i])
+                                       : (int)(row < 8 ? (uint32_t)D0[q][i] << 8 : (uint32_t)D0[q][i]);
   }
-  if (q4 == 0) *(v2i*)&red[w][16][2 * c16] = v2i{sv[0], sv[1]};
+#pragma unroll
+  for (int q = 0; q < DPL; q++)
+    if (q4 == 0) red[w][16][DPL * c16 + q] = sv[q];
   __syncthreads();
-  for (int idx = tid; idx < grp * 32; idx += 64 * NW) {
-    const int hr = idx >> 5, d = idx & 31, h = g * grp + hr;
+  for (int idx = tid; idx < grp * ND; idx += 64 * NW) {
+    const int hr = idx / ND, d = idx % ND, h = g * grp + hr;
     if (h < hb || h >= he) continue;
     uint32_t t = 0;
 #pragma unroll 4
@@ -1339,11 +1350,15 @@ hipError_t fgm_launch_attn(const AttnArgs& a, hipStream_t st) {
     else
       hipLaunchKernelGGL(attn_pv_tile_kernel<1>, grid, dim3(256), 0, st, a);
   } else {
-    const dim3 grid(a.hd / 32, a.m * a.kvh, a.p3_chunks);
-    if (grp > 8)
-      hipLaunchKernelGGL(attn_pv_kernel<true>, grid, dim3(512), 0, st, a);
+    const dim3 grid(a.hd / a.p3_dims, a.m * a.kvh, a.p3_chunks);
+    if (grp > 8 && a.p3_dims == 16)
+      hipLaunchKernelGGL((attn_pv_kernel<true, 1>), grid, dim3(512), 0, st, a);
+    else if (grp > 8)
+      hipLaunchKernelGGL((attn_pv_kernel<true, 2>), grid, dim3(512), 0, st, a);
+    else if (a.p3_dims == 16)
+      hipLaunchKernelGGL((attn_pv_kernel<false, 1>), grid, dim3(1024), 0, st, a);
     else
-      hipLaunchKernelGGL(attn_pv_kernel<false>, grid, dim3(1024), 0, st, a);
+      hipLaunchKernelGGL((attn_pv_kernel<false, 2>), grid, dim3(1024), 0, st, a);
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (a.p3_chunks > 1 || a.dup) {

@@ -149,6 +149,7 @@ struct AttnArgs {
   int32_t* part;      // P.V partial sums [m][nh][p3_chunks][hd]; before them, int8 queries [m][nh][hd]
   float* wq;          // per (row, head): query scale, then the dequantisation step (0 = zero output)
   int p1_steps;       // 64-slot steps per score workgroup
+  int p3_dims;        // dims per P.V workgroup
   int p3_steps;       // 64-slot steps per P.V workgroup
   int p3_chunks;      // P.V chunks of p3_steps
 };
