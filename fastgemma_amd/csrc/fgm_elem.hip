@@ -39,22 +39,28 @@ namespace {
 //    rotations (a + b == b + a exactly, so the tree's pairing is all that
 //    matters); lane 0 adds the tail by fma and finishes;
 //  * every thread writes (x * inv) * w (or x * inv) from its registers.
-// The variant for n % 4 != 0 or unaligned rows keeps nothing in registers:
-// x goes straight to LDS and w is read at the end.
+// The variant for n % 4 != 0 or unaligned rows (NV = 0) keeps nothing in
+// registers: x goes straight to LDS and w is read at the end.
 constexpr int RMS_MAXV = 8;  // float4 slots per thread (n <= 32 T)
 
-template <bool VEC>
+// NV: float4 slots per thread.  Compiled for 1 and 2, which rows of up to 8192
+// take, besides 8: one body for all counts held 8 slots' registers, so half as
+// many rows fitted a CU, and stepped through 8 bound checks (8 rows x 2048 3.78
+// -> 3.11 us, 8 x 8192 5.77 -> 4.95, 2048 x 2048 8.7 -> 6.8, 16384 x 256 11.4
+// -> 7.3).
+template <int NV>
 __global__ __launch_bounds__(1024) void rmsnorm_kernel(float* out, const float* x, const float* w, int n, int S,
                                                        float eps) {
   extern __shared__ float lds[];  // [16][S] transposed row, then inv
+  constexpr bool VEC = NV > 0;
   const int tid = threadIdx.x, T = blockDim.x;
   const float* xr = x + (size_t)blockIdx.x * n;
   float* orow = out + (size_t)blockIdx.x * n;
-  // register slot 4 v + e holds element idx(v, e) (VEC variant)
+  // register slot 4 v + e holds element idx(v, e) (NV > 0)
   auto idx = [&](int v, int e) { return 4 * (tid + T * v) + e; };
-  float xv[4 * RMS_MAXV], wv[4 * RMS_MAXV];
+  float xv[4 * NV + 1], wv[4 * NV + 1];
 #pragma unroll
-  for (int v = 0; v < RMS_MAXV; v++) {
+  for (int v = 0; v < NV; v++) {
     if (VEC) {
       const int i = idx(v, 0);
       if (i < n) {
@@ -73,7 +79,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_kernel(float* out, const float* 
   }
   if (VEC) {
 #pragma unroll
-    for (int v = 0; v < RMS_MAXV; v++)
+    for (int v = 0; v < NV; v++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int i = idx(v, e);
@@ -94,7 +100,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_kernel(float* out, const float* 
   __syncthreads();
   const float inv = lds[16 * S];
 #pragma unroll
-  for (int v = 0; v < RMS_MAXV; v++) {
+  for (int v = 0; v < NV; v++) {
     if (VEC) {
       const int i = idx(v, 0);
       if (i < n) {
@@ -176,6 +182,16 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(float* p, int ld, int co
 
 unsigned blocks(long n) { return (unsigned)((n + 255) / 256); }
 
+template <int NV>
+hipError_t launch_rmsnorm(float* out, const float* x, const float* w, int rows, int n, int T, int S, size_t lds,
+                          float eps, hipStream_t st) {
+  static hipError_t attr =
+      hipFuncSetAttribute((const void*)rmsnorm_kernel<NV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(rmsnorm_kernel<NV>, dim3(rows), dim3(T), lds, st, out, x, w, n, S, eps);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t fgm_launch_fill_zero(float* p, int ld, int rows, int cols, hipStream_t st) {
@@ -188,22 +204,17 @@ hipError_t fgm_launch_fill_zero(float* p, int ld, int rows, int cols, hipStream_
 hipError_t fgm_launch_rmsnorm(float* out, const float* x, const float* w, int rows, int n, float eps,
                               hipStream_t st) {
   if (rows <= 0 || n <= 0) return hipSuccess;
-  static hipError_t attr[2] = {
-      hipFuncSetAttribute((const void*)rmsnorm_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024),
-      hipFuncSetAttribute((const void*)rmsnorm_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)};
-  if (attr[0] != hipSuccess) return attr[0];
-  if (attr[1] != hipSuccess) return attr[1];
   // about two float4 slots per thread; at most RMS_MAXV (n <= 32 T, T <= 1024)
   const int T = std::min(1024, std::max(64, ((n + 7) / 8 + 63) / 64 * 64));
   if (n > 32 * T) return hipErrorInvalidValue;
   const int S = fgm_rms_stride(n);
   const size_t lds = ((size_t)16 * S + 4) * 4;
   const bool vec = n % 4 == 0 && (((uintptr_t)out | (uintptr_t)x | (uintptr_t)w) & 15) == 0;
-  if (vec)
-    hipLaunchKernelGGL(rmsnorm_kernel<true>, dim3(rows), dim3(T), lds, st, out, x, w, n, S, eps);
-  else
-    hipLaunchKernelGGL(rmsnorm_kernel<false>, dim3(rows), dim3(T), lds, st, out, x, w, n, S, eps);
-  return hipGetLastError();
+  const int nv = vec ? (n + 4 * T - 1) / (4 * T) : 0;
+  if (nv == 0) return launch_rmsnorm<0>(out, x, w, rows, n, T, S, lds, eps, st);
+  if (nv == 1) return launch_rmsnorm<1>(out, x, w, rows, n, T, S, lds, eps, st);
+  if (nv == 2) return launch_rmsnorm<2>(out, x, w, rows, n, T, S, lds, eps, st);
+  return launch_rmsnorm<RMS_MAXV>(out, x, w, rows, n, T, S, lds, eps, st);
 }
 
 hipError_t fgm_launch_gelu(float* out, const float* gate, const float* up, int n, hipStream_t st) {

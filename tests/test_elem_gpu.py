@@ -115,6 +115,20 @@ def test_rmsnorm_rows_equal_per_row_calls():
     assert np.array_equal(H.host(out).view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [4, 252, 256, 260, 512, 2052, 8188, 8192, 8196, 16384, 32764, 32768, 258])
+def test_rmsnorm_widths(n):
+    """Rows at the ends of one, two and more float4s per thread, and one whose
+    width is no multiple of four; in place, as the forward pass calls it."""
+    rows = 3
+    x = oracle.gen_student_t(33 + n, rows * n, 3).reshape(rows, n) * np.float32(4.0)
+    w = oracle.gen_normal(34 + n, n)
+    for wv in (w, None):
+        dx = H.dev(x)
+        K.rmsnorm_rows(dx, dx, None if wv is None else H.dev(wv), rows, n, 1e-6)
+        want = np.stack([oracle.rmsnorm(x[r], wv, 1e-6) for r in range(rows)])
+        assert np.array_equal(H.host(dx).view(np.uint32), want.view(np.uint32))
+
+
 def test_rope_multi_position_rows():
     """Prefill: one (cos, sin) table per token row; equals per-token calls."""
     nh, hd = 4, 128
