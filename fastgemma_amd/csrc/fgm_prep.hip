@@ -515,6 +515,7 @@ hipError_t fgm_launch_prep(const PrepBatch& in, hipStream_t st) {
   const int pre = b.count ? b.p[0].preop : PREP_COPY;
   if (pre < PREP_COPY || pre > PREP_GELU_MUL) return hipErrorInvalidValue;
   int nwg = 0, kmax = 0, lds_floats = 0;
+  long rows = 0;
   for (int i = 0; i < b.count; i++) {
     PrepProb& p = b.p[i];
     if (p.preop != pre || (pre != PREP_COPY && p.k % 64)) return hipErrorInvalidValue;
@@ -524,6 +525,7 @@ hipError_t fgm_launch_prep(const PrepBatch& in, hipStream_t st) {
       const int end = p.pa ? ((p.r1 + 15) / 16) * 16 : p.r1;
       p.nwg = end - p.r0;
       nwg = std::max(nwg, p.nwg);
+      rows += p.nwg;
       if (p.k > kmax) kmax = p.k;
       if (p.hsz > 0 && p.k > lds_floats) lds_floats = p.k;
       // the transposed row plus 1/rms (16 S + 1 > k floats)
@@ -540,6 +542,18 @@ hipError_t fgm_launch_prep(const PrepBatch& in, hipStream_t st) {
   int threads = std::min(cap, ((kmax + 3) / 4 + 63) / 64 * 64);
   threads = std::max(threads, ((kmax + 4 * VMAX - 1) / (4 * VMAX) + 63) / 64 * 64);
   threads = std::max(64, std::min(threads, PREP_MAX_THREADS));
+  // Rows whose waves would be all that the chip holds at once (32 on each of
+  // 256 CUs) or more are no longer a matter of one row's latency: half the
+  // waves, each with twice the loads in flight, launch and meet at barriers in
+  // less time (k = 2048, 1024 / 2048 rows: copy 3.90 -> 3.67 / 6.1 -> 4.7 us,
+  // rmsnorm 5.3 -> 5.0 / 8.5 -> 6.5; 768 rows of k = 1536, below the line,
+  // rmsnorm 4.27 -> 4.43).  Halved once: at a quarter, rotations get slower
+  // (hsz 512, 2048 rows 7.9 -> 8.6 us); to two float4s per thread, rmsnorm to
+  // four (k = 4096, 4096 rows: copy 14.0 -> 14.8 us, rmsnorm 21.6 -> 17.8).
+  // gelu_mul, bound by its arithmetic and memory, is the same either way.
+  const int half = (threads / 2 + 63) / 64 * 64, most = pre == PREP_COPY ? 2 : 4;
+  if (pre != PREP_GELU_MUL && rows * (threads / 64) >= 32 * 256 && ((kmax + 3) / 4 + half - 1) / half <= most)
+    threads = half;
   // the kernel has a row body for 1 .. VMAX float4s per thread only
   if (((kmax + 3) / 4 + threads - 1) / threads > VMAX) return hipErrorInvalidValue;
   const size_t lds = (size_t)lds_floats * sizeof(float);

@@ -168,3 +168,35 @@ def test_prep_rows_every_rotation_size(case):
         for g, w_, name in zip([H.host(t) for t in (drot, dqa, dqs, dpa)], want,
                                ("rot", "qa", "qs", "pa")):
             assert np.array_equal(bits(g), bits(w_)), "fused " + name
+
+
+@pytest.mark.parametrize("pre,m,k,hsz,lda", [
+    ("copy", 1008, 2048, 0, 2048),     # below the line: a float4 per thread
+    ("copy", 1023, 2048, 0, 2048),     # on it (with the pad row): two
+    ("copy", 1361, 1536, 512, 1600),   # 192 threads, a rotation through LDS
+    ("copy", 1030, 2008, 0, 2008),     # the scalar tail
+    ("rms", 1024, 2048, 128, 2048),
+    ("rms", 1366, 1344, 64, 1344),     # 192 threads, the last of them idle
+    ("rms", 1040, 4096, 1024, 4096),   # four float4s per thread
+])
+def test_prep_many_rows(pre, m, k, hsz, lda):
+    """Rows past the count at which a row gets half the threads."""
+    print(f"prep {pre} m={m} k={k} hsz={hsz} lda={lda}", flush=True)
+    t = H.torch()
+    x, w = rms_inputs(m, k, lda, 500 + m + k)
+    src = x[:, :k] if pre == "copy" else np.stack([oracle.rmsnorm(r, w, EPS) for r in x[:, :k]])
+    if k % 64:  # quantised rows alone
+        qa, qs = oracle.quant_act(src, m, k)
+        dqa, dqs = (t.full(s, 5, dtype=d, device="cuda") for s, d in (((m, k), t.int8), ((m,), t.float32)))
+        K.quant_act(H.dev(x), m, k, dqa, dqs)
+        got, want = (dqa, dqs), (qa, qs)
+    else:
+        want = oracle_prep(src, m, k, hsz)
+        _, *got = dev_outputs(m, k)
+        drot, dqa, dqs, dpa = got
+        if pre == "copy":
+            K.prep_rows(H.dev(x), lda, drot, dqa, dqs, dpa, m, k, hsz, 0, m)
+        else:
+            K.prep_rmsnorm(H.dev(x), lda, H.dev(w), EPS, dqs, dpa, m, k, hsz, rot=drot, qa=dqa)
+    for g, w_ in zip(got, want):
+        assert np.array_equal(bits(H.host(g)).reshape(-1), bits(w_).reshape(-1))
