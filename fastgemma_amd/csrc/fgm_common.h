@@ -193,6 +193,21 @@ FGM_DEV float exp16(float x) {
   return y * __int_as_float(((int)fx + 127) << 23);
 }
 
+// 1 - 2 / d for d in [1, 2^128), as exp16 and the addition of 1 leave it.  The
+// division needs none of its general form's scaling and special cases (11
+// instructions, of about 40 for a gelu): a reciprocal with one Newton step,
+// then the quotient corrected by its remainder, six.  q equals 2.0f / d for
+// every float d in [1, 2^126) and 1 - q for every one from 1 up (past 2^126
+// the reciprocal is subnormal, and 1 - q is 1), each compared on gfx950.
+// gelu_mul fused with the prep, four decode blocks of 8 rows x 8192 each:
+// 114.7 -> 113.2 us.
+FGM_DEV float one_minus_two_over(float d) {
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+  const float q = r + r;
+  return 1.0f - __builtin_fmaf(__builtin_fmaf(-d, q, 2.0f), r, q);
+}
+
 // gelu_tanh_v (ops.c:96-107) on one lane, and the scalar tail's form
 // (ops.c:114, 126; GCC fuses v + 0.044715 v^3 into one fma).  The tail's
 // tanhf is evaluated in double and rounded once.
@@ -200,7 +215,7 @@ FGM_DEV float gelu_vec(float x) {
   const float x3 = (x * x) * x;
   const float u = 0.7978845608028654f * __builtin_fmaf(0.044715f, x3, x);
   const float e = exp16(u + u);
-  const float t = 1.0f - 2.0f / (e + 1.0f);
+  const float t = one_minus_two_over(e + 1.0f);
   return (0.5f * x) * (1.0f + t);
 }
 FGM_DEV float tanh_rn(float a) { return (float)tanh((double)a); }

@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void softcap_kernel(float* x, int n, float cap
   if (i < (n & ~15)) {
     const float u = v * (1.0f / cap);
     const float e = exp16(u + u);
-    x[i] = cap * (1.0f - 2.0f / (e + 1.0f));
+    x[i] = cap * one_minus_two_over(e + 1.0f);
   } else {
     x[i] = cap * tanh_rn(v / cap);
   }
