@@ -602,7 +602,8 @@ __global__ __launch_bounds__(T_, T_ == 512 && NQ <= 4 ? 8 : 4) void attn_softmax
 // ------------------------------------------------------------------ 3. P.V
 constexpr uint32_t IW_BIAS = 32896u;  // 256 * 128 + 128: see the planes above
 
-FGM_DEV int dot4_ones(int x, int c) { return __builtin_amdgcn_sdot4(x, 0x01010101, c, false); }
+constexpr int ONES = 0x01010101;
+FGM_DEV int dot4(int x, int y, int c) { return __builtin_amdgcn_sdot4(x, y, c, false); }
 
 // Single rows.  grid (hd / (16 DPL), m * kvh, p3_chunks), 64 NW threads:
 // workgroup (x, y, z) takes the dims [16 DPL x, + 16 DPL) and the steps
@@ -666,14 +667,15 @@ __global__ __launch_bounds__(TWO ? 512 : 1024) void attn_pv_kernel(const AttnArg
       }
     }
   };
-  auto mul = [&](int i) {
+  auto mul = [&](int i, int step) {
+    const int ones = step < last ? ONES : 0;
 #pragma unroll
     for (int q = 0; q < DPL; q++) {
       const v4i b = {V[i][0][q], V[i][1][q], V[i][2][q], V[i][3][q]};
       D0[q] = mfma16(A[i][0], b, D0[q]);
       if constexpr (TWO) D1[q] = mfma16(A[i][TWO ? 1 : 0], b, D1[q]);
 #pragma unroll
-      for (int rr = 0; rr < 4; rr++) sv[q] = dot4_ones(b[rr], sv[q]);
+      for (int rr = 0; rr < 4; rr++) sv[q] = dot4(b[rr], ones, sv[q]);
     }
   };
 #pragma unroll
@@ -682,7 +684,7 @@ __global__ __launch_bounds__(TWO ? 512 : 1024) void attn_pv_kernel(const AttnArg
   for (int step = first + w; step < last; step += PF * NW) {
 #pragma unroll
     for (int i = 0; i < PF; i++) {
-      mul(i);
+      mul(i, step + i * NW);
       load(i, step + (PF + i) * NW);
     }
   }
@@ -798,7 +800,7 @@ __global__ __launch_bounds__(256 * NG, 2) void attn_pv_tile_kernel(const AttnArg
 #pragma unroll
       for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int rr = 0; rr < 4; rr++) sv[q] = dot4_ones(V[rr][q], sv[q]);
+        for (int rr = 0; rr < 4; rr++) sv[q] = dot4(V[rr][q], ONES, sv[q]);
     }
   };
 #pragma unroll

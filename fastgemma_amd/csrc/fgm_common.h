@@ -86,7 +86,9 @@ FGM_DEV int8_t quant_tail(float v) {
 // offset lies at or beyond `bytes` reads 0 without touching memory, which is
 // how the kernels mask rows and columns without branches.
 constexpr int FGM_BUF_FLAGS = 0x00020000;  // gfx9 family descriptor word 3
-constexpr uint32_t FGM_OOB = 0x80000000u;  // an offset no buffer here reaches
+// An offset past the end of every buffer here, except a K or V cache of 2 GiB or
+// more (up to 4 GiB): attention uses nothing that a masked lane read from those.
+constexpr uint32_t FGM_OOB = 0x80000000u;
 // Cache-policy operand of the buffer load / store builtins on gfx950: nt
 // (non-temporal, streamed past the caches' normal allocation).
 constexpr int FGM_CPOL_NT = 2;

@@ -204,6 +204,61 @@ def test_job_row_tiles_and_long_rows(nh, kvh, hd, cap, ring, window, pos, rows):
         same_or_tail_close(got[r], want, noncr)
 
 
+@pytest.fixture(scope="module")
+def big_cache():
+    """K and V bytes of a layer cache past 2 GiB, and its scales: views of it with
+    any kv width are valid caches."""
+    t = H.torch()
+    size = (1 << 31) + (1 << 26)
+    g = t.Generator(device="cuda").manual_seed(5)
+    kv = [t.randint(-127, 128, (size,), dtype=t.int8, device="cuda", generator=g) for _ in range(2)]
+    sc = [t.rand(size // 512, device="cuda", generator=g) * 4e-4 + 1e-4 for _ in range(2)]
+    yield size, kv[0], sc[0], kv[1], sc[1]
+    del kv, sc
+    t.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("nh,kvh,hd,nseq,rows,window,high", [
+    (8, 4, 512, 1, 1, 1500, False),   # single rows, 16 dims a workgroup
+    (8, 4, 512, 1, 1, 1500, True),    # slots past the first 2 GiB
+    (8, 4, 512, 16, 1, 1100, False),  # 32 dims a workgroup
+    (16, 1, 512, 1, 1, 700, False),   # more than eight heads
+    (16, 1, 512, 16, 1, 700, True),
+    (8, 4, 512, 1, 40, 3000, True),   # row tiles
+    (8, 4, 512, 1, 2, 300, True),     # the single-launch path
+])
+def test_caches_past_two_gib(big_cache, nh, kvh, hd, nseq, rows, window, high):
+    """Caches of 2 GiB and more hold real bytes where smaller ones read zeros."""
+    print(f"attn big cache heads {nh}/{kvh} seqs {nseq} rows {rows} high {high}", flush=True)
+    size, kc, ks, vt, vs = big_cache
+    kvd = kvh * hd
+    cap = size // kvd // 4 * 4
+    m = nseq * rows
+    q = oracle.gen_uniform(77 + m, m * nh * hd, -1.0, 1.0).reshape(m, nh * hd)
+    out = H.torch().full((m * nh * hd,), 7.0, dtype=H.torch().float32, device="cuda")
+    seqs, want = [], []
+    for i in range(nseq):
+        pos = (cap if high else 6000) - rows - 37 * i
+        seqs.append((kc, ks, vt, vs, cap, 0, pos, rows))
+        for r in range(rows):
+            if r not in (0, rows // 2, rows - 1):
+                want.append(None)
+                continue
+            en = pos + r + 1
+            st = max(en - window, 0)
+            base = st // 4 * 4
+            kv = oracle.KvLayer((en - base + 3) // 4 * 4, kvh, hd)
+            last = base + kv.cap
+            kv.kc, kv.vt = (H.host(x[base * kvd:last * kvd]) for x in (kc, vt))
+            kv.ks, kv.vs = (H.host(x[base:last]) for x in (ks, vs))
+            want.append(oracle_out("heads", q[i * rows + r], kv, nh, st - base, en - base, 0, nh, 0, 0.0))
+    K.attend(out, H.dev(q.reshape(-1)), seqs, nh, kvh, hd, window)
+    got = H.host(out).reshape(m, nh * hd)
+    for r, w in enumerate(want):
+        if w is not None:
+            same_or_tail_close(got[r], *w)
+
+
 def test_kv_store_matches_reference_write_path():
     """fgm_hip_kv_store_dev equals quant_act + store_v_t per row (the forward
     pass's write, forward.rs:515-548), linear and wrapping ring."""
