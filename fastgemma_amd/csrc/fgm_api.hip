@@ -1056,6 +1056,7 @@ static int attn_plan(AttnArgs& a, int* max_span) {
   std::fill(a.tile0, a.tile0 + FGM_ATTN_MAX_SEQ, INT_MAX);
   a.one_row = 1;
   a.dup = 0;
+  bool aligned = true;
   for (int i = 0; i < a.nseq; i++) {
     AttnSeq& s = a.seq[i];
     if (s.nrows < 0) return fail(FGM_HIP_EINVAL, "attend: sequence %d has %d rows", i, s.nrows);
@@ -1066,6 +1067,7 @@ static int attn_plan(AttnArgs& a, int* max_span) {
     s.row0 = a.row0[i] = m;
     m += s.nrows;
     a.one_row &= s.nrows == 1;
+    if (s.nrows) aligned = aligned && (((uintptr_t)s.kc | (uintptr_t)s.vc) & 3) == 0;
     for (int j = 0; j < s.nrows; j++) {
       const int en = s.pos0 + j + 1, st = attn_start(en, s.lo, a.window), n = en - st;
       if (st < 0 || n < 0)
@@ -1090,8 +1092,10 @@ static int attn_plan(AttnArgs& a, int* max_span) {
   a.max_n = mn;
   a.max_steps = steps_max;
   // Row tiles where the sequences have several rows to share K and V between
-  // (four on average), else every row by itself.
-  a.rt = m >= 4 * a.nseq ? std::max(1, FGM_ATTN_TILE / grp) : 1;
+  // (four on average), else every row by itself.  The tiles' LDS-DMA reads from
+  // dword addresses: caches at other ones take the single rows' register loads,
+  // which need no alignment.
+  a.rt = aligned && m >= 4 * a.nseq ? std::max(1, FGM_ATTN_TILE / grp) : 1;
   a.ntiles = 0;
   a.tile_steps = 1;
   for (int i = 0; i < a.nseq; i++) {

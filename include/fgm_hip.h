@@ -177,7 +177,7 @@ int fgm_hip_scale_dev(float *a, float s, int n, void *stream);
  * rounded).  Limits: head_dim a multiple of 64 up to 512, at most 16 query
  * heads per kv head, at most 32768 positions per row, a ring range no longer
  * than the ring (the reference's scratch layout assumes it too), a layer's K
- * and V caches under 4 GiB each (32-bit offsets; not checked). */
+ * and V caches under 4 GiB each (32-bit offsets; not checked), at any address. */
 
 /* drop-ins, host pointers, same parameters as the reference's symbols; the
  * caches are uploaded per call, `scratch` is not touched */

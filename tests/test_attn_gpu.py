@@ -204,6 +204,38 @@ def test_job_row_tiles_and_long_rows(nh, kvh, hd, cap, ring, window, pos, rows):
         same_or_tail_close(got[r], want, noncr)
 
 
+@pytest.mark.parametrize("shift", [1, 4, 8])
+@pytest.mark.parametrize("nh,kvh,hd,cap,ring,window,pos,rows", [
+    (8, 1, 512, 2000, 0, 0, 1960, 40),      # row tiles where the caches are at dword addresses
+    (8, 2, 128, 1300, 1300, 1200, 3000, 2), # single rows, a wrapped ring
+    (16, 1, 64, 500, 0, 0, 490, 3),
+    (8, 4, 64, 3000, 0, 1100, 2900, 100),   # row tiles of 64 dims
+    (8, 1, 256, 540, 540, 500, 3000, 6),    # the single-launch path
+])
+def test_caches_at_any_address(nh, kvh, hd, cap, ring, window, pos, rows, shift):
+    """K and V caches `shift` bytes past a 16-byte boundary, their scales one float."""
+    t = H.torch()
+    print(f"attn unaligned {shift} heads {nh}/{kvh} hd {hd} rows {rows}", flush=True)
+    q, kv = cases.attn_inputs(f"shift{rows}", nh, kvh, hd, cap, 1.0)
+
+    def moved(x, by):
+        buf = t.zeros(x.size + by, dtype=H.dev(x[:1]).dtype, device="cuda")
+        buf[by:] = H.dev(x)
+        return buf[by:]
+
+    kc, ks, vt, vs = moved(kv.kc, shift), moved(kv.ks, 1), moved(kv.vt, shift), moved(kv.vs, 1)
+    assert kc.data_ptr() % 16 == shift and vt.data_ptr() % 16 == shift
+    qrows = np.stack([np.roll(q, 17 * r) for r in range(rows)])
+    out = t.full((rows * nh * hd,), 7.0, dtype=t.float32, device="cuda")
+    K.attend(out, H.dev(qrows.reshape(-1)), [(kc, ks, vt, vs, cap, ring, pos, rows)], nh, kvh, hd, window)
+    got = H.host(out).reshape(rows, nh * hd)
+    for r in range(rows):
+        en = pos + r + 1
+        st = max(en - window, 0) if window else 0
+        want, noncr = oracle_out("heads", qrows[r], kv, nh, st, en, 0, nh, ring, 0.0)
+        same_or_tail_close(got[r], want, noncr)
+
+
 @pytest.fixture(scope="module")
 def big_cache():
     """K and V bytes of a layer cache past 2 GiB, and its scales: views of it with
