@@ -919,9 +919,9 @@ __global__ __launch_bounds__(128) void attn_final_kernel(const AttnArgs a) {
 //   E [hpw][16][S] f32 (per head, e[16 c + j] at [j][c]), reused for the
 //   int32 P.V sums [NW][3 hpw][64] | planes [blocks][3 hpw][16] int8 + one row pad.
 constexpr int FUSED_MAX_N = 1024, FUSED_MAX_GRP = 8;
-// sixteen waves while a tile's registers leave room for four waves per SIMD
-// (eight: the decode job above the same, 256 rows 15.1 -> 15.5 us)
-__host__ __device__ constexpr int fused_waves(int hd) { return hd <= 256 ? 16 : 8; }
+// most waves of a workgroup: sixteen while a tile's registers leave room for
+// four waves per SIMD
+constexpr int fused_max_waves(int hd) { return hd <= 256 ? 16 : 8; }
 
 __host__ __device__ inline int fused_stride(int n) { return (((n + 15) >> 4) + 16 + 63) / 64 * 64 + 4; }
 __host__ __device__ inline size_t fused_e_bytes(int nw, int hpw, int max_n) {
@@ -1170,9 +1170,23 @@ __global__ __launch_bounds__(64 * NW) void attn_fused_kernel(const AttnArgs a) {
   }
 }
 
-template <int KS>
+// Sixteen waves where only one workgroup shares a CU (its LDS is more than half
+// of it, or there is one for each) and has several heads' positions to walk;
+// else eight, of which two to four workgroups share one and overlap their
+// chains.  Sixteen -> eight waves: 8 heads on 4 kv heads of 128, window 64, 256
+// / 1024 rows 25.6 -> 14.4 / 93.6 -> 45.5 us; 8 on 1 of 64, a prompt of 512 rows
+// 23.7 -> 16.7; 8 decode rows, 8 on 1 of 256, window 512 12.4 -> 12.0; on the
+// other side, 256 rows of 8 heads on 1, window 1024 at head_dim 128 19.4 -> 21.2
+// and window 512 at 256 17.0 -> 17.3.
+int fused_waves(const AttnArgs& a) {
+  const int wgs = a.m * a.kvh * ((a.nh / a.kvh + a.hpw - 1) / a.hpw);
+  const bool alone = fused_lds(8, a.hd, a.hpw, a.max_n, a.max_steps) > 80 * 1024 ||
+                     (wgs <= 256 && a.hpw * a.max_n >= 3000);
+  return std::min(alone ? 16 : 8, fused_max_waves(a.hd));
+}
+
+template <int KS, int NW>
 hipError_t launch_fused(const AttnArgs& a, size_t lds, hipStream_t st) {
-  constexpr int NW = fused_waves(64 * KS);
   static hipError_t attr = hipFuncSetAttribute((const void*)attn_fused_kernel<KS, NW>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   if (attr != hipSuccess) return attr;
@@ -1322,9 +1336,13 @@ hipError_t fgm_launch_attn(const AttnArgs& a, hipStream_t st) {
   f.hpw = 1;
   while (f.hpw < grp && a.m * a.kvh * ((grp + f.hpw - 1) / f.hpw) > 256) f.hpw *= 2;
   f.hpw = std::min(f.hpw, grp);
-  const size_t flds = fused_lds(fused_waves(a.hd), a.hd, f.hpw, a.max_n, a.max_steps);
+  const int nw = fused_waves(f);
+  const size_t flds = fused_lds(nw, a.hd, f.hpw, a.max_n, a.max_steps);
   if (a.max_n <= FUSED_MAX_N && grp <= FUSED_MAX_GRP && !(fz && fz[0] == '0') && flds <= 160 * 1024)
-    return with_ks(a.hd, [&](auto ks) { return launch_fused<decltype(ks)::value>(f, flds, st); });
+    return with_ks(a.hd, [&](auto ks) {
+      constexpr int KS = decltype(ks)::value;
+      return nw == 8 ? launch_fused<KS, 8>(f, flds, st) : launch_fused<KS, fused_max_waves(64 * KS)>(f, flds, st);
+    });
 
   const int chunks = (a.tile_steps + a.p1_steps - 1) / a.p1_steps;
   if (a.rt > 1) {

@@ -204,6 +204,44 @@ def test_job_row_tiles_and_long_rows(nh, kvh, hd, cap, ring, window, pos, rows):
         same_or_tail_close(got[r], want, noncr)
 
 
+def check_job(specs, nh, kvh, hd, window, some=None):
+    """One attend call over the sequences (cap, ring, pos, rows); every row (or, of
+    a sequence of more, its first, last and `some` between) against the oracle."""
+    t = H.torch()
+    m = sum(s[3] for s in specs)
+    out = t.full((m * nh * hd,), 7.0, dtype=t.float32, device="cuda")
+    seqs, qs, rows = [], [], []
+    for i, (cap, ring, pos, n) in enumerate(specs):
+        q, kv = cases.attn_inputs(f"job{i % 3}", nh, kvh, hd, cap, 1.0)
+        seqs.append((*dev_kv(kv), cap, ring, pos, n))
+        qs.append(np.stack([np.roll(q, 17 * (r + i)) for r in range(n)]))
+        look = set(range(n)) if some is None or n <= some + 2 else {n * j // (some + 1) for j in range(some + 1)} | {n - 1}
+        rows += [(kv, ring, pos + r, qs[-1][r]) if r in look else None for r in range(n)]
+    K.attend(out, H.dev(np.concatenate([x.reshape(-1) for x in qs])), seqs, nh, kvh, hd, window)
+    got = H.host(out).reshape(m, nh * hd)
+    for r, x in enumerate(rows):
+        if x is None:
+            continue
+        kv, ring, p, q = x
+        want, noncr = oracle_out("heads", q, kv, nh, max(p + 1 - window, 0) if window else 0, p + 1, 0, nh, ring, 0.0)
+        same_or_tail_close(got[r], want, noncr)
+
+
+@pytest.mark.parametrize("nh,kvh,hd,cap,ring,window,pos,rows", [
+    (8, 8, 64, 200, 200, 64, 500, 130),      # one head per workgroup, 1040 workgroups of eight waves
+    (8, 4, 128, 200, 0, 0, 0, 200),          # a prompt from its first row, two heads
+    (4, 2, 192, 300, 300, 170, 700, 120),    # three 64-dim blocks on eight waves
+    (8, 1, 64, 1100, 1100, 1024, 3000, 40),  # two heads of 1024 positions: eight waves
+    (8, 1, 64, 1100, 1100, 1024, 3000, 70),  # four: sixteen
+    (8, 1, 256, 1200, 1200, 1024, 3000, 130),
+    (6, 2, 256, 600, 600, 520, 900, 90),     # three heads of 520 positions: eight waves
+])
+def test_job_waves_per_workgroup(nh, kvh, hd, cap, ring, window, pos, rows):
+    """The single launch at both its widths, full and partly filled CUs."""
+    print(f"attn waves rows {rows} heads {nh}/{kvh} hd {hd} window {window}", flush=True)
+    check_job([(cap, ring, pos, rows)], nh, kvh, hd, window, some=20)
+
+
 @pytest.mark.parametrize("shift", [1, 4, 8])
 @pytest.mark.parametrize("nh,kvh,hd,cap,ring,window,pos,rows", [
     (8, 1, 512, 2000, 0, 0, 1960, 40),      # row tiles where the caches are at dword addresses
