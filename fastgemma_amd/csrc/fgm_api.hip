@@ -1036,8 +1036,8 @@ void fgm_softcap_hip(float* x, int n, float cap) { DROPIN(dropin_softcap(x, n, c
 
 // ------------------------------------------------------ int8-KV attention
 // Validates the sequences, fills the row bookkeeping and the grid of `a`
-// (scratch pointers excepted); *max_n, *max_span receive the longest range
-// and the longest range-or-ring of any row.
+// (scratch pointers excepted); *max_span receives the longest range or ring of
+// any row.
 static int attn_plan(AttnArgs& a, int* max_span) {
   if (a.nh <= 0 || a.kvh <= 0 || a.nh % a.kvh)
     return fail(FGM_HIP_EINVAL, "attend: n_heads=%d is not a multiple of kv_heads=%d", a.nh, a.kvh);
@@ -1052,6 +1052,7 @@ static int attn_plan(AttnArgs& a, int* max_span) {
   if (!a.out || !a.q) return fail(FGM_HIP_EINVAL, "attend: out or q is NULL");
   const int grp = a.nh / a.kvh;
   int m = 0, mn = 0, ms = 1, steps_max = 1;
+  long long row_steps = 0;
   std::fill(a.row0, a.row0 + FGM_ATTN_MAX_SEQ, INT_MAX);
   std::fill(a.tile0, a.tile0 + FGM_ATTN_MAX_SEQ, INT_MAX);
   a.one_row = 1;
@@ -1085,28 +1086,47 @@ static int attn_plan(AttnArgs& a, int* max_span) {
       mn = std::max(mn, n);
       ms = std::max(ms, std::max(n, s.ring));
       steps_max = std::max(steps_max, sp.dom_steps);
+      row_steps += sp.dom_steps;
       a.dup |= sp.lo0 < sp.hi1;
     }
   }
   a.m = m;
   a.max_n = mn;
   a.max_steps = steps_max;
-  // Row tiles where the sequences have several rows to share K and V between
-  // (four on average), else every row by itself.  The tiles' LDS-DMA reads from
-  // dword addresses: caches at other ones take the single rows' register loads,
-  // which need no alignment.
-  a.rt = aligned && m >= 4 * a.nseq ? std::max(1, FGM_ATTN_TILE / grp) : 1;
-  a.ntiles = 0;
-  a.tile_steps = 1;
-  for (int i = 0; i < a.nseq; i++) {
-    AttnSeq& s = a.seq[i];
-    a.tile0[i] = a.ntiles;
-    a.ntiles += (s.nrows + a.rt - 1) / a.rt;
-    for (int j = 0; j < s.nrows; j += a.rt) {
-      const int st = attn_start(s.pos0 + j + 1, s.lo, a.window), en = s.pos0 + std::min(j + a.rt, s.nrows);
-      a.tile_steps = std::max(a.tile_steps, attn_span(st, en, s.ring, s.ring ? st % s.ring : st).dom_steps);
+  // Row tiles or every row by itself, for the call as a whole.  By themselves
+  // rows read their 64-slot steps of K and V each (128 head_dim bytes a kv head)
+  // at close to the memory's rate; a tile reads the steps of its rows' union once,
+  // but at about half that rate (four waves stage each step for one CU), stores
+  // its scores for 128 pairs, and the queries take a launch.  So tiles from 32 MB
+  // of single-row reads beyond twice the tiles': measured both ways on 1094 jobs
+  // (1 to 16 sequences of 1 to 512 rows, decode rows beside a prefill chunk, 100
+  // to 32000 positions, 1 to 16 heads a kv head), the choice costs 0.8 % over the
+  // faster side on average; four rows a sequence as the line cost 5.5 %.  Single /
+  // tiles, 8 heads on one kv head of 512: 4 rows of 1500 positions 20 / 28 us,
+  // 12 of 8192 39 / 39, 24 of 8192 54 / 41; 15 decode rows and a chunk of 49 at
+  // 8192 93 / 82, at 2048 50 / 45; 12 sequences of 2 rows at 8192 60 / 62.
+  // The tiles' LDS-DMA reads from dword addresses: caches at other ones take the
+  // single rows' register loads, which need no alignment.
+  auto tile = [&](int rt) {
+    a.rt = rt;
+    a.ntiles = 0;
+    a.tile_steps = 1;
+    long long steps = 0;
+    for (int i = 0; i < a.nseq; i++) {
+      AttnSeq& s = a.seq[i];
+      a.tile0[i] = a.ntiles;
+      a.ntiles += (s.nrows + rt - 1) / rt;
+      for (int j = 0; j < s.nrows; j += rt) {
+        const int st = attn_start(s.pos0 + j + 1, s.lo, a.window), en = s.pos0 + std::min(j + rt, s.nrows);
+        const int n = attn_span(st, en, s.ring, s.ring ? st % s.ring : st).dom_steps;
+        a.tile_steps = std::max(a.tile_steps, n);
+        steps += n;
+      }
     }
-  }
+    return steps;
+  };
+  const int rt = std::max(1, FGM_ATTN_TILE / grp);
+  if (!aligned || (row_steps - 2 * tile(rt)) * a.kvh * a.hd * 128 < 32000000) tile(1);
   // 64-slot steps per score workgroup: about 512 workgroups
   const long long units = std::max(1, a.ntiles * a.kvh);
   a.p1_steps = (int)std::max<long long>(1, std::min<long long>(8, (a.tile_steps * units + 511) / 512));

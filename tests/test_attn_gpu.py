@@ -214,10 +214,10 @@ def check_job(specs, nh, kvh, hd, window, some=None):
     for i, (cap, ring, pos, n) in enumerate(specs):
         q, kv = cases.attn_inputs(f"job{i % 3}", nh, kvh, hd, cap, 1.0)
         seqs.append((*dev_kv(kv), cap, ring, pos, n))
-        qs.append(np.stack([np.roll(q, 17 * (r + i)) for r in range(n)]))
+        qs.append([np.roll(q, 17 * (r + i)) for r in range(n)])
         look = set(range(n)) if some is None or n <= some + 2 else {n * j // (some + 1) for j in range(some + 1)} | {n - 1}
         rows += [(kv, ring, pos + r, qs[-1][r]) if r in look else None for r in range(n)]
-    K.attend(out, H.dev(np.concatenate([x.reshape(-1) for x in qs])), seqs, nh, kvh, hd, window)
+    K.attend(out, H.dev(np.concatenate([x for rs in qs for x in rs])), seqs, nh, kvh, hd, window)
     got = H.host(out).reshape(m, nh * hd)
     for r, x in enumerate(rows):
         if x is None:
@@ -240,6 +240,57 @@ def test_job_waves_per_workgroup(nh, kvh, hd, cap, ring, window, pos, rows):
     """The single launch at both its widths, full and partly filled CUs."""
     print(f"attn waves rows {rows} heads {nh}/{kvh} hd {hd} window {window}", flush=True)
     check_job([(cap, ring, pos, rows)], nh, kvh, hd, window, some=20)
+
+
+@pytest.mark.parametrize("name,nh,kvh,hd,window,specs", [
+    # a chunk beside 15 decode rows: below and past the line from which rows go in tiles
+    ("rows", 8, 1, 512, 0, [(1300, 0, 1299 - 9 * i, 1) for i in range(15)] + [(1400, 0, 1365, 30)]),
+    ("tiles", 8, 1, 512, 0, [(1300, 0, 1299 - 9 * i, 1) for i in range(15)] + [(1500, 0, 1430, 61)]),
+    ("tiles", 8, 4, 128, 1100, [(1204, 1204, 3000 + 301 * i, 1) for i in range(3)] + [(1204, 1204, 2500, 100)]),
+    # a few rows in each sequence, one without any
+    ("rows", 8, 2, 256, 0, [(1200, 0, 1100 + i, 2 + i) for i in range(5)] + [(64, 0, 0, 0)]),
+    ("rows", 16, 1, 256, 0, [(700, 0, 600, 7), (100, 0, 3, 1), (90, 0, 0, 90)]),
+    ("tiles", 16, 1, 256, 0, [(700, 0, 300, 400), (100, 0, 3, 1), (90, 0, 0, 90)]),
+    # tiles of 42 rows: 126 of the 128 pairs; the last one partial, tails at every offset
+    ("tiles", 3, 1, 128, 0, [(1400, 0, 1200, 130)]),
+    ("tiles", 8, 1, 64, 0, [(3000, 0, 2860, 130)]),
+    # wrapped rings: both runs in one slot group; a gap between them
+    ("tiles", 16, 1, 256, 1498, [(1500, 1500, 4000, 70)]),
+    ("tiles", 8, 2, 192, 1100, [(2100, 2100, 2090, 60)]),
+])
+def test_job_rows_or_tiles(name, nh, kvh, hd, window, specs):
+    """Mixed jobs on both sides of the choice between single rows and row tiles."""
+    print(f"attn {name} heads {nh}/{kvh} hd {hd} rows {[s[3] for s in specs]}", flush=True)
+    check_job(specs, nh, kvh, hd, window, some=12)
+
+
+@pytest.mark.parametrize("nh,kvh,hd,cap,rows", [
+    (8, 1, 64, 1500, 33),    # 256 or more (row, head) pairs, 1 .. 4 and 6 groups of slots a thread
+    (8, 1, 64, 4000, 33),
+    (8, 1, 64, 5200, 33),
+    (8, 1, 64, 8192, 33),
+    (8, 1, 64, 12200, 33),
+    (8, 1, 64, 20500, 33),
+    (8, 1, 64, 3000, 2),     # fewer: 1, 2, 3, 4, 6 and 9 groups, twice the threads
+    (8, 1, 64, 8000, 2),
+    (8, 1, 64, 12200, 2),
+    (8, 1, 64, 15000, 2),
+    (8, 1, 64, 24000, 2),
+    (8, 1, 64, 32768, 2),
+])
+def test_job_softmax_widths(nh, kvh, hd, cap, rows):
+    """Every width of the softmax, by row length and (row, head) pairs."""
+    print(f"attn softmax rows {rows} positions {cap}", flush=True)
+    check_job([(cap, 0, cap - rows, rows)], nh, kvh, hd, 0, some=2)
+
+
+@pytest.mark.parametrize("nh,kvh,hd", [(8, 1, 512), (9, 1, 512), (8, 2, 512), (16, 1, 512), (8, 4, 128)])
+def test_job_sixteen_decode_rows(nh, kvh, hd):
+    """Sixteen sequences of one row past the single-launch path: 32 dims a
+    workgroup in P.V, up to and past eight heads a kv head."""
+    print(f"attn decode 16 heads {nh}/{kvh} hd {hd}", flush=True)
+    check_job([(1300, 0, 1299 - 11 * i, 1) if i % 2 else (1300, 1300, 2000 + 97 * i, 1) for i in range(16)], nh, kvh, hd,
+              1290)
 
 
 @pytest.mark.parametrize("shift", [1, 4, 8])
