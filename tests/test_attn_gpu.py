@@ -265,6 +265,9 @@ def test_job_rows_or_tiles(name, nh, kvh, hd, window, specs):
 
 
 @pytest.mark.parametrize("nh,kvh,hd,cap,rows", [
+    (16, 1, 64, 64, 20),     # up to 1024 slots: 256 threads
+    (9, 1, 64, 1000, 30),
+    (12, 1, 64, 1024, 2),
     (8, 1, 64, 1500, 33),    # 256 or more (row, head) pairs, 1 .. 4 and 6 groups of slots a thread
     (8, 1, 64, 4000, 33),
     (8, 1, 64, 5200, 33),
