@@ -446,9 +446,12 @@ __global__ __launch_bounds__(256, 2) void attn_scores_tile_kernel(const AttnArgs
 // wait for their own barriers, loads and ordered sum about half the time
 // (2048 pairs x 8192: 72 us walking LDS, 42 us from registers with three
 // workgroups per CU and 54 VALU instructions a slot; 35 us with four, the V
-// scales loaded after the exponentials to fit their registers, and fewer
-// instructions).
-FGM_DEV int exp_stride(int n) { return (((n + 15) >> 4) + 16 + 63) / 64 * 64 + 4; }
+// scales loaded after the exponentials, and fewer instructions).  Four leave 64
+// registers, of which NQ = 4 is 13 short and NQ = 3 three: 56 and 16 bytes of
+// scratch a lane.
+// The row stride of the transposed exponentials, for the kernels and for the
+// LDS that their launches ask for.
+__host__ __device__ inline int exp_stride(int n) { return (((n + 15) >> 4) + 16 + 63) / 64 * 64 + 4; }
 
 template <int NQ, int T_>  // up to 512 threads, NQ <= 4: 32 waves per CU (64 registers)
 __global__ __launch_bounds__(T_, T_ <= 512 && NQ <= 4 ? 8 : 4) void attn_softmax_kernel(const AttnArgs a) {
@@ -923,9 +926,8 @@ constexpr int FUSED_MAX_N = 1024, FUSED_MAX_GRP = 8;
 // four waves per SIMD
 constexpr int fused_max_waves(int hd) { return hd <= 256 ? 16 : 8; }
 
-__host__ __device__ inline int fused_stride(int n) { return (((n + 15) >> 4) + 16 + 63) / 64 * 64 + 4; }
 __host__ __device__ inline size_t fused_e_bytes(int nw, int hpw, int max_n) {
-  const size_t e = (size_t)hpw * 16 * fused_stride(max_n) * 4, red = (size_t)nw * 3 * hpw * 64 * 4;
+  const size_t e = (size_t)hpw * 16 * exp_stride(max_n) * 4, red = (size_t)nw * 3 * hpw * 64 * 4;
   return e > red ? e : red;
 }
 // the last block's operand reads run to row 31 of 16 bytes
@@ -948,7 +950,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fused_kernel(const AttnArgs a) {
   const int hb = max(a.h0, hf), he = min(a.h1, hf + nhl);
   if (hb >= he) return;
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-  const int n = max(G.n, 0), n16 = n & ~15, S = fused_stride(n);
+  const int n = max(G.n, 0), n16 = n & ~15, S = exp_stride(n);
   int8_t* qq = (int8_t*)sm;
   float* qsc = (float*)(sm + 16 * QROW);
   float* wqs = qsc + 16;    // per head: wmax / 65535, 0 = zero output
@@ -1278,8 +1280,7 @@ hipError_t launch_softmax(const AttnArgs& a, hipStream_t st) {
   // with hundreds of (row, head) pairs several workgroups share a CU; a few
   // get the widest workgroups
   const bool many = a.m * (a.h1 - a.h0) >= 256 && quads <= 6 * 512;
-  const int S = (((a.max_n + 15) >> 4) + 16 + 63) / 64 * 64 + 4;
-  const size_t lds = ((size_t)16 * S + 32) * 4;
+  const size_t lds = ((size_t)16 * exp_stride(a.max_n) + 32) * 4;
   // up to 1024 slots: every further wave is launched and waited for without any
   // (window 64, 16 heads of 256 on one kv head: 16 rows 23.3 -> 13.3 us, 256
   // 55.6 -> 37.4; of 64: 1024 rows 131.4 -> 70.2)
