@@ -13,6 +13,8 @@
 //                   traffic figures (its algorithmic bytes are known exactly)
 //   fgm_ceil_mfma   independent int8 MFMA chains on every SIMD: the dense int8
 //                   peak (v_mfma_i32_32x32x32_i8 or v_mfma_i32_16x16x64_i8)
+//   fgm_ceil_divide  no floor: compares 1 - 2 / d as gelu and softcap compute it
+//                   with the division itself, over a range of floats d
 //   fgm_ceil_gridbar  a device-wide barrier between dependent steps inside one
 //                   cooperative launch (what a persistent decode kernel would
 //                   pay per dependent GEMM instead of a kernel boundary), with
@@ -113,6 +115,18 @@ __global__ __launch_bounds__(256) void mfma_kernel(int iters, int* sink) {
       for (int r = 0; r < 4; r++) s ^= acc[c][r];
     if (s == 0x13572468) sink[blockIdx.x] = s;
   }
+}
+
+// The floats with bit patterns [from, to) whose one_minus_two_over differs from
+// 1 - 2 / d.
+__global__ __launch_bounds__(256) void divide_kernel(uint32_t from, uint32_t to, uint32_t* differ) {
+  const uint32_t stride = gridDim.x * 256;
+  uint32_t bad = 0;
+  for (uint64_t i = (uint64_t)from + blockIdx.x * 256 + threadIdx.x; i < to; i += stride) {
+    const float d = __uint_as_float((uint32_t)i);
+    bad += __float_as_uint(one_minus_two_over(d)) != __float_as_uint(1.0f - 2.0f / d);
+  }
+  if (bad) atomicAdd(differ, bad);
 }
 
 // Device-wide barrier variants (one wave per workgroup arrives; the others
@@ -287,6 +301,13 @@ int fgm_ceil_mfma(int shape, int nwg, int iters, int* sink, void* stream) {
     hipLaunchKernelGGL(mfma_kernel<true>, dim3(nwg), dim3(256), 0, (hipStream_t)stream, iters, sink);
   else
     hipLaunchKernelGGL(mfma_kernel<false>, dim3(nwg), dim3(256), 0, (hipStream_t)stream, iters, sink);
+  return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+// differ: one word, the count is added
+int fgm_ceil_divide(uint32_t from, uint32_t to, uint32_t* differ, void* stream) {
+  if (!differ) return 1;
+  hipLaunchKernelGGL(divide_kernel, dim3(4096), dim3(256), 0, (hipStream_t)stream, from, to, differ);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

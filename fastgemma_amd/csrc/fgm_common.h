@@ -198,9 +198,9 @@ FGM_DEV float exp16(float x) {
 // 1 - 2 / d for d in [1, 2^128), as exp16 and the addition of 1 leave it.  The
 // division needs none of its general form's scaling and special cases (11
 // instructions, of about 40 for a gelu): a reciprocal with one Newton step,
-// then the quotient corrected by its remainder, six.  q equals 2.0f / d for
-// every float d in [1, 2^126) and 1 - q for every one from 1 up (past 2^126
-// the reciprocal is subnormal, and 1 - q is 1), each compared on gfx950.
+// then the quotient corrected by its remainder, six.  The result equals
+// 1.0f - 2.0f / d for every float in that range (past 2^126 the reciprocal is
+// subnormal, and the result 1): tests/test_elem_gpu.py compares them all.
 // gelu_mul fused with the prep, four decode blocks of 8 rows x 8192 each:
 // 114.7 -> 113.2 us.
 FGM_DEV float one_minus_two_over(float d) {

@@ -12,6 +12,7 @@ tail bound is stated on the term before cancellation: |got - want| <= 4 ulp of
 """
 from __future__ import annotations
 
+import ctypes as C
 import hashlib
 import json
 import os
@@ -19,6 +20,7 @@ import os
 import numpy as np
 import pytest
 
+import fastgemma_amd as F
 import oracle
 from fastgemma_amd import kernels as K
 from tests.golden import cases
@@ -88,6 +90,43 @@ def test_elementwise_device_matches_oracle_and_reference(n):
     assert sha(a) == gold["mul"]
     (a,) = gpu(lambda x: K.scale(x, 0.7071067811865476), e["x"])
     assert sha(a) == gold["scale"]
+
+
+def test_one_minus_two_over_every_float():
+    """gelu's and softcap's 1 - 2 / d against the division, for all d in [1, 2^128)."""
+    L = C.CDLL(os.path.join(os.path.dirname(F.__file__), "libfgm_ceil.so"))
+    t = H.torch()
+
+    def differ(first, end):
+        n = t.zeros(1, dtype=t.int32, device="cuda")
+        rc = L.fgm_ceil_divide(C.c_uint32(first), C.c_uint32(end), C.c_void_p(n.data_ptr()),
+                               C.c_void_p(t.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        return int(H.host(n)[0])
+
+    assert differ(0x3F800000, 0x7F800000) == 0
+    assert differ(0x00000001, 0x00800000) > 0  # subnormal d, outside the range, is where they part
+
+
+@pytest.mark.parametrize("cap", [1.0, 30.0])
+def test_softcap_and_gelu_over_the_whole_range(cap):
+    """Every exponent that exp reaches, both of its clamps, and the special values."""
+    x = np.concatenate([np.linspace(-50, 50, (1 << 20) - 16, dtype=np.float32),
+                        np.array([0.0, -0.0, 1e-45, -1e-45, 1e-30, -1e-6, 88, -88, 44, -44, 3e38, -3e38, np.inf, -np.inf,
+                                  np.nan, 1.0], np.float32)])
+
+    def same(got, want):
+        nan = np.isnan(want)
+        assert np.array_equal(nan, np.isnan(got))
+        assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+    with np.errstate(over="ignore"):
+        xc = x * np.float32(cap)
+    (got,) = gpu(lambda v: K.softcap(v, cap), xc)
+    same(got, oracle.softcap(xc, cap))
+    g = x * np.float32(0.25) if cap == 1.0 else x
+    (got,) = gpu(K.gelu, g)
+    same(got, oracle.gelu_mul(g, None))
 
 
 @pytest.mark.parametrize("nh,hd,pos", cases.ROPE_CASES)
