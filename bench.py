@@ -1,6 +1,6 @@
 """Benchmark of the fgm-kernels quantized-matmul path on one MI355X.
 
-    python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-extra] [--no-cpu]
+    python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-extra] [--no-cpu] [--json FILE]
 
 Headline workload: batched decode skinny GEMM,
 M = 8 activation rows ~ N(0,1) fp32, int4 weights group 64 with f16 scales,
@@ -905,13 +905,17 @@ class CpuPath:
                                 N, 1, P(self.t1))
 
 
-def time_cpu(fn, min_reps=10, min_s=0.3):
+def time_cpu(fn, min_reps=10, min_s=0.3, max_s=2.0):
     """fn timed after one warm-up call: at least min_reps calls and min_s
-    seconds; (median, min, max, reps) in seconds, as fgm-bench main.rs:190-199
-    reports them."""
+    seconds, but no call past max_s seconds after the first; (median, min, max,
+    reps) in seconds, as fgm-bench main.rs:190-199 reports them.  (The port's
+    M = 2048 calls take about 5 s each.)"""
     fn()
-    ts, t_end = [], time.perf_counter() + min_s
-    while len(ts) < min_reps or time.perf_counter() < t_end:
+    ts, t_start = [], time.perf_counter()
+    while True:
+        t = time.perf_counter() - t_start
+        if ts and ((len(ts) >= min_reps and t >= min_s) or t >= max(min_s, max_s)):
+            break
         t0 = time.perf_counter()
         fn()
         ts.append(time.perf_counter() - t0)
@@ -945,6 +949,7 @@ def cpu_configs(cp):
                 (rng.random((K // 64) * N, dtype=np.float32) * 0.045 + 0.005).astype(np.float16).view(np.uint16))
 
     out = {}
+    log("cpu cfg1")
     # cfg1: int8 GEMV M=1
     a = cp.act(1, 2048, 31)
     W = w8(8192, 2048)
@@ -953,6 +958,7 @@ def cpu_configs(cp):
     out["cfg1"] = {"gemm": _rec(time_cpu(lambda: cp.gemm(8, a, 8192, *W, c)), b, "GB/s"),
                    "prep_gemm": _rec(time_cpu(lambda: (cp.prep(a), cp.gemm(8, a, 8192, *W, c))),
                                      b + prep_bytes(1, 2048), "GB/s")}
+    log("cpu cfg3")
     # cfg3: the seven M=256 int8 projections, and the layer
     acts = {K: cp.act(256, K, 40 + K) for K in (2048, 8192)}
     r3, lay_g, lay_pg = {}, [], []
@@ -975,6 +981,7 @@ def cpu_configs(cp):
                    "prep_gemm": _rec(time_cpu(lambda: layer(True), 5), lops, "TOPS")}
     out["cfg3"] = r3
     del ws, cs
+    log("cpu cfg4")
     # cfg4: 30 layers (q,k,v,o,gate,up int4 g64, down int8) + int8 LM head,
     # distinct buffers, M=8, the forward pass's GEMM sequence
     layers = [{name: (w8(N, K) if name == "down" else w4(N, K)) for name, N, K in LAYER} for _ in range(30)]
@@ -1001,6 +1008,7 @@ def cpu_configs(cp):
     out["cfg4"] = {"gemm": _rec(time_cpu(lambda: step(False), 5, 0.2), allb, "GB/s"),
                    "prep_gemm": _rec(time_cpu(lambda: step(True), 5, 0.2), allb + preps, "GB/s")}
     del layers, head
+    log("cpu cfg5")
     # cfg5: M=2048 heavy-tailed (gate/up int4 g64, down int8)
     r5 = {}
     x5 = {K: cp.act(2048, K, 60 + K) for K in (2048, 8192)}
@@ -1179,6 +1187,8 @@ def main():
     ap.add_argument("--only", default=None,
                     help="run one extra measurement (ceilings, cfg1, int4_stream, cfg3, vendor, sweep, cfg5, cfg4, "
                          "elem, prep_fused, attn, model, cpu) and print its JSON instead of the headline line")
+    ap.add_argument("--json", default=None,
+                    help="also write the whole record, every measurement in full, to this file")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) > 1:
         print("bench.py measures one GPU: this build has no multi-GPU path "
@@ -1275,6 +1285,14 @@ def main():
     }
     out["summary"] = summary(out)
     log("done")
+    if args.json:
+        with open(args.json, "w") as f:
+            json.dump(out, f)
+    # the line itself stays short enough to be read from the end of a log: the
+    # headline and the summary, without each measurement's own record
+    del out["extra"]
+    if cpu:
+        out["cpu_baseline"] = {k: v for k, v in cpu.items() if k not in ("per_config", "load")}
     print(json.dumps(out))
 
 
