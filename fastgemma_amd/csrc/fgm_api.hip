@@ -1054,7 +1054,6 @@ static int attn_plan(AttnArgs& a, int* max_span) {
   int m = 0, mn = 0, ms = 1, steps_max = 1;
   long long row_steps = 0;
   std::fill(a.row0, a.row0 + FGM_ATTN_MAX_SEQ, INT_MAX);
-  std::fill(a.tile0, a.tile0 + FGM_ATTN_MAX_SEQ, INT_MAX);
   a.one_row = 1;
   a.dup = 0;
   bool aligned = true;
@@ -1107,26 +1106,31 @@ static int attn_plan(AttnArgs& a, int* max_span) {
   // 8192 93 / 82, at 2048 50 / 45; 12 sequences of 2 rows at 8192 60 / 62.
   // The tiles' LDS-DMA reads from dword addresses: caches at other ones take the
   // single rows' register loads, which need no alignment.
-  auto tile = [&](int rt) {
-    a.rt = rt;
-    a.ntiles = 0;
-    a.tile_steps = 1;
+  a.rt = 1;
+  a.ntiles = m;
+  a.tile_steps = std::max(1, steps_max);
+  std::copy(a.row0, a.row0 + FGM_ATTN_MAX_SEQ, a.tile0);
+  const long long step_bytes = 128ll * a.kvh * a.hd, least = 32000000;
+  if (aligned && row_steps * step_bytes >= least) {
+    const int rt = std::max(1, FGM_ATTN_TILE / grp);
+    int tile0[FGM_ATTN_MAX_SEQ], ntiles = 0, longest = 1;
     long long steps = 0;
     for (int i = 0; i < a.nseq; i++) {
-      AttnSeq& s = a.seq[i];
-      a.tile0[i] = a.ntiles;
-      a.ntiles += (s.nrows + rt - 1) / rt;
+      const AttnSeq& s = a.seq[i];
+      tile0[i] = ntiles;
+      ntiles += (s.nrows + rt - 1) / rt;
       for (int j = 0; j < s.nrows; j += rt) {
         const int st = attn_start(s.pos0 + j + 1, s.lo, a.window), en = s.pos0 + std::min(j + rt, s.nrows);
         const int n = attn_span(st, en, s.ring, s.ring ? st % s.ring : st).dom_steps;
-        a.tile_steps = std::max(a.tile_steps, n);
+        longest = std::max(longest, n);
         steps += n;
       }
     }
-    return steps;
-  };
-  const int rt = std::max(1, FGM_ATTN_TILE / grp);
-  if (!aligned || (row_steps - 2 * tile(rt)) * a.kvh * a.hd * 128 < 32000000) tile(1);
+    if ((row_steps - 2 * steps) * step_bytes >= least) {
+      a.rt = rt, a.ntiles = ntiles, a.tile_steps = longest;
+      std::copy(tile0, tile0 + a.nseq, a.tile0);
+    }
+  }
   // 64-slot steps per score workgroup: about 512 workgroups
   const long long units = std::max(1, a.ntiles * a.kvh);
   a.p1_steps = (int)std::max<long long>(1, std::min<long long>(8, (a.tile_steps * units + 511) / 512));
