@@ -561,9 +561,10 @@ hipError_t fgm_launch_gemm(int bits, const GemmBatch& in, hipStream_t st) {
     return bnt ? launch_any<8, 1, 1, 2, 1, 4, 1, 4, false, true>(in, st) : launch_any<8, 1, 1, 2, 1, 4, 1, 4>(in, st);
   }
   // int4 is bound by VALU issue, and the matrix cores' cycles come on top of it
-  // (70 % and 23 % of the cycles on the 128x128 tile of 64x64 waves): 128x32
+  // (65 % and 22 % of the cycles on the 128x128 tile of 64x64 waves): 128x32
   // waves unpack each B dword once per workgroup instead of twice (M = 2048,
-  // N = 8192, K = 2048, gate + up: 134 -> 124 us).
+  // N = 8192, K = 2048: 25.0 -> 22.4 M VALU instructions, 63 % and 24 %, 64.4 ->
+  // 58.3 us a dispatch; gate + up in one launch 134 -> 124 us).
   if (tiles(in, 128, 128) >= 480) return launch_any<4, 4, 1, 1, 4, 2, 2>(in, st);
   if (tiles(in, 128, 64) >= 240) return launch_any<4, 2, 1, 2, 2, 2, 2>(in, st);
   return launch_any<4, 1, 1, 2, 1, 4, 2>(in, st);
