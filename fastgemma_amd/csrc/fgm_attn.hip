@@ -1175,11 +1175,11 @@ __global__ __launch_bounds__(64 * NW) void attn_fused_kernel(const AttnArgs a) {
 // Sixteen waves where only one workgroup shares a CU (its LDS is more than half
 // of it, or there is one for each) and has several heads' positions to walk;
 // else eight: two such workgroups share a CU (at 122 registers it holds sixteen
-// waves) and overlap their chains.  Sixteen -> eight waves: 8 heads on 4 kv heads of 128, window 64, 256
-// / 1024 rows 25.6 -> 14.4 / 93.6 -> 45.5 us; 8 on 1 of 64, a prompt of 512 rows
-// 23.7 -> 16.7; 8 decode rows, 8 on 1 of 256, window 512 12.4 -> 12.0; on the
-// other side, 256 rows of 8 heads on 1, window 1024 at head_dim 128 19.4 -> 21.2
-// and window 512 at 256 17.0 -> 17.3.
+// waves) and overlap their chains.  Sixteen -> eight waves: 8 heads on 4 kv heads
+// of 128, window 64, 256 / 1024 rows 25.6 -> 14.4 / 93.6 -> 45.5 us; 8 on 1 of 64,
+// a prompt of 512 rows 23.7 -> 16.7; 8 decode rows, 8 on 1 of 256, window 512
+// 12.4 -> 12.0; on the other side, 256 rows of 8 heads on 1, window 1024 at
+// head_dim 128 19.4 -> 21.2 and window 512 at 256 17.0 -> 17.3.
 int fused_waves(const AttnArgs& a) {
   const int wgs = a.m * a.kvh * ((a.nh / a.kvh + a.hpw - 1) / a.hpw);
   const bool alone = fused_lds(8, a.hd, a.hpw, a.max_n, a.max_steps) > 80 * 1024 ||
